@@ -1,0 +1,89 @@
+"""f32 causal GQA prefill on the fp32 matrix cores, against the oracle's sequential f32 loops.
+
+The sums run in another order than the oracle's and the exponentials in base 2; outputs are
+weighted means of V ~ N(0, 1), so the bound is 1e-5 absolute, that of the single-head f32
+kernel (tests/test_gpu_ops.py, test_attention_f32_shapes)."""
+import numpy as np
+import pytest
+
+import tilers_hip as th
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+D = th.TileDtype
+
+
+def put(dev, stream, x, offset=0):
+    b = dev.alloc(x.size + offset, D.F32)
+    b.copy_from_host(np.concatenate([np.zeros(offset, np.float32), x.reshape(-1)]), stream)
+    return b
+
+
+def prefill(dev, stream, q, k, v, B, S, start, max_seq, Dh, NH, NKV, offset=0):
+    bufs = [put(dev, stream, x, offset) for x in (q, k, v)]
+    ob = put(dev, stream, np.full(q.size, 7.0, np.float32), offset)
+    th.attention_prefill(*(b.as_raw_ptr() + 4 * offset for b in bufs + [ob]), B, S, start, max_seq,
+                         Dh, NH, NKV, D.F32, stream)
+    return ob.copy_to_host(stream)[offset:].reshape(q.shape)
+
+
+def inputs(rng, B, S, max_seq, Dh, NH, NKV):
+    return (rng.standard_normal((B, S, NH, Dh)).astype(np.float32),
+            rng.standard_normal((B, NKV, max_seq, Dh)).astype(np.float32),
+            rng.standard_normal((B, NKV, max_seq, Dh)).astype(np.float32))
+
+
+@pytest.mark.parametrize("Dh", [64, 128])
+@pytest.mark.parametrize("B,S,start,extra,NH,NKV", [
+    (1, 1, 0, 0, 2, 2),        # one query, one position
+    (3, 1, 5, 2, 4, 4),        # one query after a few cached positions
+    (1, 31, 0, 0, 4, 2),       # less than one 32-query group
+    (1, 33, 31, 1, 4, 1),      # a second group of one query; diagonal off the block edges
+    (2, 64, 0, 0, 8, 2),       # one whole query block and stage
+    (1, 65, 64, 0, 4, 4),      # one query over, start on a stage edge
+    (2, 300, 37, 3, 8, 8),     # 16 (batch, kv head) units on 8 XCDs: grouped work order
+    (1, 257, 1000, 60, 4, 1),  # a chunk after cached positions, rows past it not read
+])
+def test_prefill_f32_shapes(dev, stream, Dh, B, S, start, extra, NH, NKV):
+    rng = np.random.default_rng(S * 7 + start + Dh)
+    max_seq = start + S + extra
+    q, k, v = inputs(rng, B, S, max_seq, Dh, NH, NKV)
+    if extra:
+        k[:, :, start + S:] = v[:, :, start + S:] = np.nan   # never written by a program
+    got = prefill(dev, stream, q, k, v, B, S, start, max_seq, Dh, NH, NKV)
+    ref = orc.attention_prefill(q, k, v, orc.F32, B, S, start, max_seq, Dh, NH, NKV)
+    err = np.abs(got - ref.reshape(q.shape)).max()
+    assert err < 1e-5, f"max err {err:.3e}"
+
+
+def test_prefill_f32_unaligned_views(dev, stream):
+    """Views 4 bytes off 16-byte alignment stay on the general kernel."""
+    rng = np.random.default_rng(11)
+    q, k, v = inputs(rng, 1, 70, 90, 64, 4, 2)
+    got = prefill(dev, stream, q, k, v, 1, 70, 20, 90, 64, 4, 2, offset=1)
+    ref = orc.attention_prefill(q, k, v, orc.F32, 1, 70, 20, 90, 64, 4, 2)
+    assert np.abs(got - ref.reshape(q.shape)).max() < 1e-5
+
+
+@pytest.mark.parametrize("Dh", [64, 128])
+@pytest.mark.parametrize("pos", [0, 40, 69, 99])
+def test_prefill_f32_later_positions_do_not_reach_a_query(dev, stream, Dh, pos):
+    """NaN and infinities at position `pos` of K and V: queries before it are those of the
+    finite inputs bit for bit, whatever stage and block `pos` shares with them; a query that
+    sees an infinite V value has it in that column."""
+    rng = np.random.default_rng(pos + Dh)
+    q, k, v = inputs(rng, 1, 100, 100, Dh, 2, 1)
+    clean = prefill(dev, stream, q, k, v, 1, 100, 0, 100, Dh, 2, 1)
+    for kind in ("k nan", "v nan", "v inf"):
+        kb, vb = k.copy(), v.copy()
+        if kind == "k nan":
+            kb[:, :, pos, 3] = np.nan
+        else:
+            vb[:, :, pos, 5] = np.nan if kind == "v nan" else np.inf
+        got = prefill(dev, stream, q, kb, vb, 1, 100, 0, 100, Dh, 2, 1)
+        assert np.array_equal(got[:, :pos], clean[:, :pos]), kind
+        if kind != "k nan":
+            seen = got[:, pos:, :, 5]
+            assert (np.isnan(seen) if kind == "v nan" else seen == np.inf).all(), kind
+            rest = np.delete(got[:, pos:], 5, axis=3)
+            assert np.array_equal(rest, np.delete(clean[:, pos:], 5, axis=3)), kind

@@ -1,7 +1,7 @@
 // Attention kernels: GQA decode (split-KV, MFMA scores), a general online-softmax
 // kernel for every other shape/dtype, and the constants and work order of the
-// causal GQA prefill (its kernel is in prefill_asm.hpp, f32 single-head attention
-// in attention_f32.hpp).
+// causal GQA prefill (its 16-bit kernel is in prefill_asm.hpp; f32 single-head
+// attention and f32 prefill are in attention_f32.hpp).
 //
 // Semantics (reference):
 //   prefill  __tile_attention_prefill_f32  crates/tile_std/src/tile.rs:2136, :3064;
@@ -423,7 +423,7 @@ attn_decode_combine(const float* __restrict__ ws, uint16_t* __restrict__ O, uint
 // General attention: any head_dim <= 256, any dtype (f32 / f16 / bf16), causal
 // or not.  One 256-thread workgroup per (batch, query, head); KV streamed in
 // chunks of 1024 scores kept in LDS, online softmax across chunks.  Used for
-// shapes outside the fast kernels and for the f32 single-head op.
+// shapes outside the fast kernels.
 //   kv_visible(q) = causal ? min(start_pos + q + 1, kv_len) : kv_len
 // Q and O are [B][S][NH][D] (token-major) or, with head_major, [B][NH][S][D];
 // kv tensors are [B][NKV][max_seq][D].

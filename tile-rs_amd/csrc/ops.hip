@@ -475,6 +475,27 @@ int th_attention_prefill(const void* q, const void* k, const void* v, void* o, u
     }
     return TH_OK;
   }
+  if (dtype == TH_F32 && (head_dim == 64 || head_dim == 128) && vec16) {
+    // f32: the fp32 MFMA flash kernel (every other head dim, and views off 16-byte
+    // alignment, stay on the general kernel)
+    const uint64_t blocks =
+        static_cast<uint64_t>((seq_len + th::pf32::BQ - 1) / th::pf32::BQ) * batch * num_heads;
+    if (blocks > 0x7fffffffu) return fail(TH_KERNEL_ERROR, "attention_prefill: grid too large");
+    const dim3 grid(static_cast<uint32_t>(blocks)), block(th::pf32::NT);
+    auto Q = static_cast<const float*>(q);
+    auto K = static_cast<const float*>(k);
+    auto V = static_cast<const float*>(v);
+    auto O = static_cast<float*>(o);
+    if (head_dim == 64)
+      hipLaunchKernelGGL(th::attn_prefill_f32<64>, grid, block, 0, as_stream(s), Q, K, V, O, batch,
+                         seq_len, start_pos, max_seq, num_heads, num_kv_heads,
+                         scale * th::kLog2e);
+    else
+      hipLaunchKernelGGL(th::attn_prefill_f32<128>, grid, block, 0, as_stream(s), Q, K, V, O,
+                         batch, seq_len, start_pos, max_seq, num_heads, num_kv_heads,
+                         scale * th::kLog2e);
+    return launch_status("attention_prefill (fp32 MFMA) launch");
+  }
   return attn_general_launch(q, k, v, o, batch, seq_len, start_pos, max_seq, start_pos + seq_len,
                              head_dim, num_heads, num_kv_heads, 1, scale, dtype, as_stream(s));
 }
