@@ -1,4 +1,4 @@
-"""f32 causal GQA prefill on the fp32 matrix cores, against the oracle's sequential f32 loops.
+"""f32 causal GQA prefill and GQA decode on the fp32 matrix cores, against the oracle's sequential f32 loops.
 
 The sums run in another order than the oracle's and the exponentials in base 2; outputs are
 weighted means of V ~ N(0, 1), so the bound is 1e-5 absolute, that of the single-head f32
@@ -87,3 +87,35 @@ def test_prefill_f32_later_positions_do_not_reach_a_query(dev, stream, Dh, pos):
             assert (np.isnan(seen) if kind == "v nan" else seen == np.inf).all(), kind
             rest = np.delete(got[:, pos:], 5, axis=3)
             assert np.array_equal(rest, np.delete(clean[:, pos:], 5, axis=3)), kind
+
+
+@pytest.mark.parametrize("B,L,extra,NH,NKV,Dh,ws", [
+    (1, 1, 0, 4, 4, 128, "none"),       # one position
+    (3, 513, 7, 16, 1, 128, "full"),    # G = 16, chunk boundary + 1, rows past L not read
+    (2, 1024, 0, 8, 8, 128, "none"),    # G = 1, whole chunks
+    (1, 9000, 40, 8, 1, 64, "full"),    # G = 8, head_dim 64, 18 splits
+    (2, 4500, 0, 4, 2, 128, "part"),    # a workspace that holds fewer records than the plan
+    (2, 4500, 0, 4, 2, 128, "tiny"),    # one too small for any split
+    (64, 700, 0, 32, 8, 64, "none"),    # 512 items: unsplit
+    (1, 200, 0, 6, 2, 128, "none"),     # G = 3: the general kernel
+])
+def test_decode_f32_shapes(dev, stream, B, L, extra, NH, NKV, Dh, ws):
+    rng = np.random.default_rng(L * 3 + NH)
+    max_seq = L + extra
+    q = rng.standard_normal((B, NH, Dh)).astype(np.float32)
+    k, v = (rng.standard_normal((B, NKV, max_seq, Dh)).astype(np.float32) for _ in range(2))
+    k[:, :, L:] = v[:, :, L:] = np.nan
+    bufs = [put(dev, stream, x) for x in (q, k, v)]
+    ob = put(dev, stream, np.full(q.size, 7.0, np.float32))
+    rec = B * NH * (Dh + 2) * 4
+    size = {"none": 0, "full": th.attention_decode_workspace_size(B, L, Dh, NH, NKV),
+            "part": 5 * rec, "tiny": rec + 8}[ws]
+    # a guard after the workspace shows a write past it
+    wb = put(dev, stream, np.full(size // 4 + 1024, 3.0, np.float32)) if size else None
+    th.attention_decode(*bufs, ob, B, L, max_seq, Dh, NH, NKV, D.F32, wb, size, stream)
+    got = ob.copy_to_host(stream).reshape(q.shape)
+    ref = orc.attention_decode(q, k, v, orc.F32, B, L, max_seq, Dh, NH, NKV)
+    err = np.abs(got - ref.reshape(q.shape)).max()
+    assert err < 1e-5, f"max err {err:.3e}"
+    if wb is not None:
+        assert (wb.copy_to_host(stream)[size // 4:] == 3.0).all()

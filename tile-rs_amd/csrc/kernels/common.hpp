@@ -60,6 +60,12 @@ __device__ __forceinline__ uint16_t f32_to_u16(float f) {
   else return f32_to_f16(f);
 }
 
+template <int DT, class T>
+__device__ __forceinline__ void store_elem(T* p, float v) {
+  if constexpr (DT == kF32) *p = v;
+  else *p = f32_to_u16<DT>(v);
+}
+
 // Two f32 -> packed pair of 16-bit values (lo in bits 0..15).
 template <int DT>
 __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
@@ -176,6 +182,21 @@ __device__ __forceinline__ f32x4 mfma16x16x32(u32x4 a, u32x4 b, f32x4 c) {
   } else {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
                                                    __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  }
+}
+
+// 16 x 16 MFMA step over one 16-byte fragment per lane of both operands: 32 k values in
+// 16 bits, 16 in f32 (four 16x16x4, whose lane group g takes k value 4 g + j in step j).
+template <int DT>
+__device__ __forceinline__ f32x4 mfma16x16(u32x4 a, u32x4 b, f32x4 c) {
+  if constexpr (DT == kF32) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      c = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a[j]), __uint_as_float(b[j]), c, 0,
+                                               0, 0);
+    return c;
+  } else {
+    return mfma16x16x32<DT>(a, b, c);
   }
 }
 

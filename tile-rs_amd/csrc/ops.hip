@@ -504,6 +504,12 @@ static uint32_t decode_chunks(uint32_t seq_len) {
   return (seq_len + th::dec::CHUNK - 1) / th::dec::CHUNK;
 }
 
+// At most `most` splits of whole chunks, none of them empty.
+static void decode_split_cap(uint32_t nchunks, uint32_t most, uint32_t* n_split, uint32_t* cps) {
+  *cps = (nchunks + most - 1) / most;
+  *n_split = (nchunks + *cps - 1) / *cps;
+}
+
 // KV split of the decode: about two workgroups per CU in total (measured on
 // MI355X: config 5's 512 (batch, kv_head) items run fastest unsplit, 332 us
 // against 350 us with one workgroup per chunk; a single item at 32K positions
@@ -511,15 +517,12 @@ static uint32_t decode_chunks(uint32_t seq_len) {
 static void decode_plan(uint32_t items, uint32_t nchunks, uint32_t* n_split, uint32_t* cps) {
   const uint32_t target = 2 * current_cu_count();
   uint32_t n = (target + items - 1) / items;
-  n = std::max(1u, std::min(n, nchunks));
-  *cps = (nchunks + n - 1) / n;
-  *n_split = (nchunks + *cps - 1) / *cps;
+  decode_split_cap(nchunks, std::max(1u, std::min(n, nchunks)), n_split, cps);
 }
 
 // The MFMA decode: head_dim 128 or 64 (both native), G = 1..16 query heads per kv head.
-static bool decode_fast(uint32_t head_dim, uint32_t nh, uint32_t nkv, th_dtype dtype) {
-  if (dtype == TH_F32 || (head_dim != th::dec::D && head_dim != 64) || nkv == 0 || nh % nkv != 0)
-    return false;
+static bool decode_fast(uint32_t head_dim, uint32_t nh, uint32_t nkv) {
+  if ((head_dim != th::dec::D && head_dim != 64) || nkv == 0 || nh % nkv != 0) return false;
   const uint32_t g = nh / nkv;
   return g == 1 || g == 2 || g == 4 || g == 8 || g == 16;
 }
@@ -542,11 +545,11 @@ static void decode_split_launch(const void* q, const void* k, const void* v, voi
                                 uint32_t batch, uint32_t seq_len, uint32_t max_seq, uint32_t nh,
                                 uint32_t nkv, uint32_t n_split, uint32_t cps, float sl2,
                                 hipStream_t s) {
+  using T = th::elem_t<DT>;
   const dim3 grid(batch * nkv * n_split), block(th::dec::NT);
   hipLaunchKernelGGL((th::attn_decode_split<DT, G, HD>), grid, block, 0, s,
-                     static_cast<const uint16_t*>(q), static_cast<const uint16_t*>(k),
-                     static_cast<const uint16_t*>(v), static_cast<uint16_t*>(o), ws, seq_len,
-                     max_seq, nh, nkv, n_split, cps, sl2);
+                     static_cast<const T*>(q), static_cast<const T*>(k), static_cast<const T*>(v),
+                     static_cast<T*>(o), ws, seq_len, max_seq, nh, nkv, n_split, cps, sl2);
 }
 
 template <int DT, int HD>
@@ -608,21 +611,20 @@ static void decode_run_hd(const void* Q, const void* K, const void* V, void* O, 
                           uint32_t num_kv_heads, uint32_t n_split, uint32_t cps, float sl2,
                           th_dtype dtype, hipStream_t s) {
   const uint32_t g = num_heads / num_kv_heads;
-  if (dtype == TH_BF16)
-    decode_launch_g<th::kBF16, HD>(g, Q, K, V, O, ws, batch, seq_len, max_seq, num_heads,
-                                   num_kv_heads, n_split, cps, sl2, s);
-  else
-    decode_launch_g<th::kF16, HD>(g, Q, K, V, O, ws, batch, seq_len, max_seq, num_heads,
-                                  num_kv_heads, n_split, cps, sl2, s);
-  // with one split each workgroup covered its whole sequence and wrote O
-  if (n_split > 1) {
-    const dim3 cgrid(batch * num_heads), cblock(th::dec::CT);
-    if (dtype == TH_BF16)
-      hipLaunchKernelGGL((th::attn_decode_combine<th::kBF16, HD>), cgrid, cblock, 0, s, ws,
-                         static_cast<uint16_t*>(O), num_heads, num_kv_heads, n_split);
-    else
-      hipLaunchKernelGGL((th::attn_decode_combine<th::kF16, HD>), cgrid, cblock, 0, s, ws,
-                         static_cast<uint16_t*>(O), num_heads, num_kv_heads, n_split);
+  auto go = [&](auto dt) {
+    constexpr int DT = decltype(dt)::value;
+    decode_launch_g<DT, HD>(g, Q, K, V, O, ws, batch, seq_len, max_seq, num_heads, num_kv_heads,
+                            n_split, cps, sl2, s);
+    // with one split each workgroup covered its whole sequence and wrote O
+    if (n_split > 1)
+      hipLaunchKernelGGL((th::attn_decode_combine<DT, HD>), dim3(batch * num_heads),
+                         dim3(th::dec::CT), 0, s, ws, static_cast<th::elem_t<DT>*>(O), num_heads,
+                         num_kv_heads, n_split);
+  };
+  switch (dtype) {
+    case TH_F32: go(std::integral_constant<int, th::kF32>{}); break;
+    case TH_F16: go(std::integral_constant<int, th::kF16>{}); break;
+    default: go(std::integral_constant<int, th::kBF16>{}); break;
   }
 }
 
@@ -647,9 +649,9 @@ extern "C" {
 static bool decode_pad(const void* q, const void* k, const void* v, const void* o,
                        uint32_t head_dim, uint32_t num_heads, uint32_t num_kv_heads,
                        th_dtype dtype) {
-  return head_dim < th::dec::D && head_dim % 8 == 0 &&
-         decode_fast(th::dec::D, num_heads, num_kv_heads, dtype) && aligned16(q) &&
-         aligned16(k) && aligned16(v) && aligned16(o);
+  return dtype != TH_F32 && head_dim < th::dec::D && head_dim % 8 == 0 &&
+         decode_fast(th::dec::D, num_heads, num_kv_heads) && aligned16(q) && aligned16(k) &&
+         aligned16(v) && aligned16(o);
 }
 
 int th_attention_decode(const void* q, const void* k, const void* v, void* o, uint32_t batch,
@@ -670,7 +672,7 @@ int th_attention_decode(const void* q, const void* k, const void* v, void* o, ui
     return th::check_hip(hipMemsetAsync(o, 0, bytes, as_stream(s)), "hipMemsetAsync",
                          TH_MEMORY_ERROR);
   }
-  const bool fast = decode_fast(head_dim, num_heads, num_kv_heads, dtype) && aligned16(q) &&
+  const bool fast = decode_fast(head_dim, num_heads, num_kv_heads) && aligned16(q) &&
                     aligned16(k) && aligned16(v);
   // Other head dims below 128 (multiples of 8): Q and the live rows of K and V (the first
   // seq_len of each (batch, kv_head)) are copied zero-padded to 128 columns into the
@@ -723,7 +725,23 @@ int th_attention_decode(const void* q, const void* k, const void* v, void* o, ui
   const size_t need = th_attention_decode_workspace_size(batch, seq_len, th::dec::D, num_heads,
                                                          num_kv_heads);
   void* ws = workspace;
-  if (ws) {
+  if (dtype == TH_F32) {
+    // A workspace is never required for f32: the split uses the caller's as far as it
+    // reaches, else the stream's scratch, else (no memory, or a capture, whose replays
+    // could meet on that scratch) each item runs unsplit.
+    const size_t rec = static_cast<size_t>(batch) * num_heads * (head_dim + 2) * sizeof(float);
+    if (ws && n_split > 1 && workspace_bytes / rec < n_split) {
+      const uint32_t fit = static_cast<uint32_t>(workspace_bytes / rec);
+      if (fit >= 2) decode_split_cap(decode_chunks(seq_len), fit, &n_split, &cps);
+      else ws = nullptr;
+    }
+    if (!ws && n_split > 1 &&
+        (stream_capturing(as_stream(s)) ||
+         th::stream_scratch(as_stream(s), n_split * rec, &ws) != TH_OK)) {
+      ws = nullptr;
+      decode_split_cap(decode_chunks(seq_len), 1, &n_split, &cps);
+    }
+  } else if (ws) {
     if (workspace_bytes < need)
       return fail(TH_MEMORY_ERROR, "attention_decode: workspace of " +
                                        std::to_string(workspace_bytes) + " bytes < required " +
@@ -764,8 +782,9 @@ int th_attention_decode_static(const void* q, const void* k, const void* v, void
                        static_cast<unsigned char*>(o), bytes);
     return launch_status("attention_decode_static zero");
   }
-  const bool fast = decode_fast(head_dim, num_heads, num_kv_heads, dtype) && aligned16(q) &&
-                    aligned16(k) && aligned16(v);
+  // (f32 stays on the general kernel, which shares no array between overlapping calls)
+  const bool fast = dtype != TH_F32 && decode_fast(head_dim, num_heads, num_kv_heads) &&
+                    aligned16(q) && aligned16(k) && aligned16(v);
   if (!fast) {
     // th_attention_decode would pad these shapes into allocated copies; every other
     // shape it runs on the general kernel, which needs no scratch

@@ -43,5 +43,15 @@ inline uint32_t current_cu_count() {
   return n;
 }
 
+// Whether work enqueued on `s` is being recorded into a graph.
+inline bool stream_capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return st != hipStreamCaptureStatusNone;
+}
+
 }  // namespace ops
 }  // namespace th
