@@ -168,4 +168,189 @@ gemm_f32_mfma(const float* __restrict__ A, const float* __restrict__ B, void* __
       up ? static_cast<const char*>(up) + co : nullptr);
 }
 
+// ============================================================================
+// 64 x 64 tiles, for products whose 128 x 128 tiles would leave CUs idle.
+//
+// Bound: the fp32 matrix cores, once every SIMD has work.  999 x 4096 x 1000 is 64 tiles
+// of 128 x 128 (a quarter of the chip, one wave per SIMD there) and 256 of 64 x 64.  Eight
+// waves per workgroup, two per SIMD: wave (kh, wm, wn) computes 32 x 32 of the tile over
+// half kh of every 64-deep K stage, and the two halves' sums are added through LDS at the
+// end.  Two LDS stages; the next stage's values wait in registers while the current one
+// computes.  A product with fewer tiles still is also split over K (grid z), f32 partials to
+// a workspace that gemm_splitk_reduce adds in order.
+//
+// LDS holds A^T[k][m] and B[k][n], rows of 64 floats, column x of row k at
+// x ^ 32 (k & 1) ^ 16 ((k >> 2) & 3): the two k rows of an MFMA operand read fall in
+// opposite halves of the 64 banks, and so do (4 rows of 16 columns) the transposing
+// writes, whose 16 lane groups then read 64 consecutive bytes of a matrix row each.
+//
+// Measured on MI355X: 999 x 4096 x 1000 522 -> 91 us (90 TFLOP/s), 1024^3 96 -> 27,
+// 300 x 3000 x 500 397 -> 21, 64 x 4096 x 64 427 -> 10.
+// ============================================================================
+namespace gf32s {
+constexpr int BM = 64, BN = 64, BK = 64;
+constexpr int NT = 512;
+using gf32::f32x16;
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// Values c .. c + 3 of a row of `cols`, zeros from `cols` on, without a branch on the lane
+// and in two parts: fetch4 loads (a piece past the end reads the row's last four values),
+// fix4 then makes the piece of what was loaded, so that only fix4 waits for the load.
+// VEC: 16-byte aligned rows and cols % 4 == 0 (a piece is all inside or all outside).
+template <bool VEC>
+__device__ __forceinline__ f32x4 fetch4(const float* __restrict__ row, uint32_t c, uint32_t cols) {
+  if constexpr (VEC) return *reinterpret_cast<const f32x4*>(row + min(c, cols - 4));
+  if (cols >= 4) return *reinterpret_cast<const f32x4u*>(row + min(c, cols - 4));
+  return f32x4{row[0], row[min(1u, cols - 1)], row[min(2u, cols - 1)], 0.0f};
+}
+template <bool VEC>
+__device__ __forceinline__ f32x4 fix4(f32x4 w, uint32_t c, uint32_t cols) {
+  if constexpr (VEC) return c < cols ? w : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  // w holds values first .. first + 3 of the row
+  const uint32_t first = cols >= 4 ? min(c, cols - 4) : 0u, sh = c - first;
+  f32x4 v;
+  v[0] = sh == 0 ? w[0] : sh == 1 ? w[1] : sh == 2 ? w[2] : sh == 3 ? w[3] : 0.0f;
+  v[1] = sh == 0 ? w[1] : sh == 1 ? w[2] : sh == 2 ? w[3] : 0.0f;
+  v[2] = sh == 0 ? w[2] : sh == 1 ? w[3] : 0.0f;
+  v[3] = sh == 0 ? w[3] : 0.0f;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) v[j] = c + j < cols ? v[j] : 0.0f;
+  return v;
+}
+
+struct alignas(16) Lds {
+  float a[2][BK * BM];
+  float b[2][BK * BN];
+};
+}  // namespace gf32s
+
+// Tile (tm, tn) of C = A . B over k in [k0, k1); other arguments as gemm_f32_tile_128.
+template <int DT_OUT, bool B_TRANS, bool VEC, int EPI>
+__device__ __forceinline__ void gemm_f32_tile_64(const float* __restrict__ A,
+                                                 const float* __restrict__ B,
+                                                 void* __restrict__ C, uint32_t M, uint32_t N,
+                                                 uint32_t K, uint32_t k0, uint32_t k1, uint32_t tm,
+                                                 uint32_t tn, const void* __restrict__ up) {
+  using namespace gf32s;
+  __shared__ Lds s;
+  const int t = threadIdx.x, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int kh = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1;
+  const int h = lane >> 5, l32 = lane & 31;
+  const uint32_t m0 = tm * BM, n0 = tn * BN;
+
+  // Staging, two 16-byte pieces per thread and operand.  K-contiguous operands: piece i is
+  // row tr, k 4 (tk + 8 i) .. +3; row-major B: k row bk + 32 i, columns 4 (lane % 16) .. +3.
+  const int tr = 16 * (wave & 3) + (lane >> 2), tk = (lane & 3) + 4 * (wave >> 2);
+  const int bk = 4 * wave + (lane >> 4), bn = 4 * (lane & 15);
+  // Rows past M (N) read the last row (columns past N zeros): they reach only outputs that
+  // are not stored.  Values past k1 are zero in both operands.
+  const float* arow = A + static_cast<size_t>(min(m0 + tr, M - 1)) * K;
+  const float* brow = B + static_cast<size_t>(min(n0 + tr, N - 1)) * K;   // B_TRANS
+  f32x4 ra[2], rb[2];
+  auto load = [&](uint32_t kb) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      ra[i] = fetch4<VEC>(arow, kb + 4 * (tk + 8 * i), k1);
+      if constexpr (B_TRANS) rb[i] = fetch4<VEC>(brow, kb + 4 * (tk + 8 * i), k1);
+      else
+        rb[i] = fetch4<VEC>(B + static_cast<size_t>(min(kb + bk + 32 * i, k1 - 1)) * N, n0 + bn, N);
+    }
+  };
+  const int tw = 256 * tk + (tr ^ (16 * (lane & 3)));   // row 4 tk, its column of tr
+  auto put = [&](float* dst, const f32x4& v, int i) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) dst[(tw ^ (32 * (j & 1))) + 64 * j + 2048 * i] = v[j];
+  };
+  auto store = [&](int buf, uint32_t kb) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint32_t kc = kb + 4 * (tk + 8 * i), kr = kb + bk + 32 * i;
+      put(s.a[buf], fix4<VEC>(ra[i], kc, k1), i);
+      if constexpr (B_TRANS) put(s.b[buf], fix4<VEC>(rb[i], kc, k1), i);
+      else
+        *reinterpret_cast<f32x4*>(
+            &s.b[buf][64 * (bk + 32 * i) + (bn ^ (32 * (bk & 1)) ^ (16 * (wave & 3)))]) =
+            kr < k1 ? fix4<VEC>(rb[i], n0 + bn, N) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+  };
+
+  f32x16 acc;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+  // operand reads: k = 32 kh + 2 ks + h, (k >> 2) & 3 = (ks >> 1) & 3
+  const int ko = 64 * (32 * kh + h);
+  const int ao = ko + ((32 * wm + l32) ^ (32 * h)), bo = ko + ((32 * wn + l32) ^ (32 * h));
+
+  const uint32_t nk = (k1 - k0 + BK - 1) / BK;
+  load(k0);
+  store(0, k0);
+  if (nk > 1) load(k0 + BK);
+  __syncthreads();
+  for (uint32_t kt = 0; kt < nk; ++kt) {
+    const int cur = kt & 1;
+    // the next stage goes into the idle buffer, and the one after it is loaded, before this
+    // stage's MFMAs: nothing but the barrier follows them
+    if (kt + 1 < nk) store(cur ^ 1, k0 + (kt + 1) * BK);
+    if (kt + 2 < nk) load(k0 + (kt + 2) * BK);
+    const float* sa = s.a[cur];
+    const float* sb = s.b[cur];
+    // operands of two MFMAs (k rows 2 apart) per group, one group ahead of their use
+    float fa[2], fb[2];
+    auto frag = [&](int g) {
+      const int x = 16 * (g & 3);
+      fa[0] = sa[(ao ^ x) + 256 * g];
+      fa[1] = sa[(ao ^ x) + 256 * g + 128];
+      fb[0] = sb[(bo ^ x) + 256 * g];
+      fb[1] = sb[(bo ^ x) + 256 * g + 128];
+    };
+    frag(0);
+#pragma unroll
+    for (int g = 0; g < BK / 8; ++g) {
+      const float a0 = fa[0], a1 = fa[1], b0 = fb[0], b1 = fb[1];
+      if (g + 1 < BK / 8) frag(g + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b0, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b1, acc, 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();
+  }
+
+  // add the two K halves: each wave hands its partner the 8 accumulators that the partner
+  // stores (accumulator r: row 8 (r / 4) + 4 h + r % 4, column l32)
+  float* x = s.a[0];
+#pragma unroll
+  for (int r = 0; r < 8; ++r) x[(8 * wave + r) * 64 + lane] = kh ? acc[r] : acc[8 + r];
+  __syncthreads();
+  const uint32_t col = n0 + 32 * wn + l32;
+#pragma unroll
+  for (int r = 0; r < 8; ++r) {
+    const float v = (kh ? acc[8 + r] : acc[r]) + x[(8 * (wave ^ 4) + r) * 64 + lane];
+    const uint32_t row = m0 + 32 * wm + 16 * kh + 8 * (r >> 2) + 4 * h + (r & 3);
+    if (row < M && col < N)
+      gemm::store_out<EPI, DT_OUT>(C, up, static_cast<size_t>(row) * N + col, v);
+  }
+}
+
+// Library kernel: tiles in XCD-aware grouped order, batch = blockIdx.y (element strides sa,
+// sb, sc), K slice = blockIdx.z: k [z ks, (z + 1) ks) to C + z M N (ks a multiple of 64; one
+// slice: ks >= K).
+template <int DT_OUT, bool B_TRANS, bool VEC, int EPI = 0>
+__global__ void __launch_bounds__(gf32s::NT)
+gemm_f32_64(const float* __restrict__ A, const float* __restrict__ B, void* __restrict__ C,
+            uint32_t M, uint32_t N, uint32_t K, uint64_t sa, uint64_t sb, uint64_t sc,
+            const void* __restrict__ up, uint32_t ks) {
+  constexpr int OSZ = (DT_OUT == kF32) ? 4 : 2;
+  uint32_t tm, tn;
+  gemm::tile_coords<gf32::GROUP_M>(blockIdx.x, (M + gf32s::BM - 1) / gf32s::BM,
+                                   (N + gf32s::BN - 1) / gf32s::BN, tm, tn);
+  const size_t co = (static_cast<size_t>(blockIdx.y) * sc +
+                     static_cast<size_t>(blockIdx.z) * M * N) * OSZ;
+  const uint32_t k0 = blockIdx.z * ks;
+  gemm_f32_tile_64<DT_OUT, B_TRANS, VEC, EPI>(
+      A + blockIdx.y * sa, B + blockIdx.y * sb, static_cast<char*>(C) + co, M, N, K, k0,
+      min(K - k0, ks) + k0, tm, tn, up ? static_cast<const char*>(up) + co : nullptr);
+}
+
 }  // namespace th

@@ -1,5 +1,5 @@
 // GEMM entry points of the C ABI (include/tilers_hip.h, section 2): th_matmul and
-// th_matmul_silu_mul.  Shapes and pointers are checked on the host, the hand-written
+// th_matmul_silu_mul, and their kernels for 16-bit operands (f32: ops_gemm_f32.hip).  Shapes and pointers are checked on the host, the hand-written
 // gfx950 kernel for the shape is picked and enqueued on the caller's stream; there is
 // no CPU fallback.  (Its own translation unit: the GEMM instantiations compile in
 // parallel with the rest of the library.)
@@ -12,8 +12,7 @@
 #include "kernels/common.hpp"
 #include "kernels/gemm.hpp"
 #include "kernels/gemm_asm.hpp"
-#include "kernels/gemm_f32.hpp"
-#include "ops_common.hpp"
+#include "ops_gemm.hpp"
 
 using th::fail;
 using namespace th::ops;
@@ -21,20 +20,6 @@ using namespace th::ops;
 namespace {
 
 // ---- matmul -------------------------------------------------------------------
-
-// One GEMM launch: C[i] = epilogue(A[i] . B[i]) for i < batch, element strides
-// sa, sb, sc; `up` (epilogue kEpiSiluMul) has C's dtype, layout and strides.
-struct GemmArgs {
-  const void* a;
-  const void* b;
-  void* c;
-  const void* up;
-  uint32_t m, k, n;
-  bool bt;
-  uint32_t batch;
-  uint64_t sa, sb, sc;
-  hipStream_t s;
-};
 
 // The LDS-DMA pipeline serves every shape with K % 32 == 0 unless
 // TILERS_HIP_GEMM_DMA=0 (a debugging switch: the register-staged kernel then
@@ -94,11 +79,8 @@ int gemm_splitk(const GemmArgs& g, uint32_t tiles, uint32_t S) {
   else if (g.m <= 64) go(std::integral_constant<int, 2>{});
   else go(std::integral_constant<int, 4>{});
   TH_TRY(launch_status("matmul (split-K) launch"));
-  const uint32_t blocks = static_cast<uint32_t>(
-      std::min<uint64_t>((mn + 255) / 256, 4ull * current_cu_count()));
-  hipLaunchKernelGGL((th::gemm_splitk_reduce<DTO, EPI>), dim3(blocks), dim3(256), 0, g.s, W, g.c,
-                     g.up, mn, S);
-  return launch_status("matmul (split-K merge) launch");
+  return splitk_merge(g, W, S,
+                      DTO == th::kF32 ? TH_F32 : DTO == th::kF16 ? TH_F16 : TH_BF16, EPI);
 }
 
 template <int DT, int DTO, int EPI, bool BT>
@@ -142,31 +124,10 @@ int gemm_mfma_go(const GemmArgs& g, dim3 grid) {
 
 template <int DT, int DTO, int EPI>
 int gemm_launch(const GemmArgs& g, bool mfma) {
-  if constexpr (DT != th::kF32) {
-    if (mfma) {
-      const dim3 grid(((g.m + 255) / 256) * ((g.n + 255) / 256), g.batch);
-      return g.bt ? gemm_mfma_go<DT, DTO, EPI, true>(g, grid)
-                  : gemm_mfma_go<DT, DTO, EPI, false>(g, grid);
-    }
-  }
-  (void)mfma;
-  if constexpr (DT == th::kF32) {
-    // the fp32 MFMA kernel; 16-byte loads when every row start is 16-byte aligned
-    const bool vec = aligned16(g.a) && aligned16(g.b) && g.k % 4 == 0 && (g.bt || g.n % 4 == 0) &&
-                     g.sa % 4 == 0 && g.sb % 4 == 0;
-    const dim3 grid(((g.m + th::gf32::BM - 1) / th::gf32::BM) * ((g.n + th::gf32::BN - 1) / th::gf32::BN),
-                    g.batch),
-        block(th::gf32::NT);
-    auto A = static_cast<const float*>(g.a);
-    auto B = static_cast<const float*>(g.b);
-    if (g.bt) {
-      if (vec) hipLaunchKernelGGL((th::gemm_f32_mfma<DTO, true, true, EPI>), grid, block, 0, g.s, A, B, g.c, g.m, g.n, g.k, g.sa, g.sb, g.sc, g.up);
-      else hipLaunchKernelGGL((th::gemm_f32_mfma<DTO, true, false, EPI>), grid, block, 0, g.s, A, B, g.c, g.m, g.n, g.k, g.sa, g.sb, g.sc, g.up);
-    } else {
-      if (vec) hipLaunchKernelGGL((th::gemm_f32_mfma<DTO, false, true, EPI>), grid, block, 0, g.s, A, B, g.c, g.m, g.n, g.k, g.sa, g.sb, g.sc, g.up);
-      else hipLaunchKernelGGL((th::gemm_f32_mfma<DTO, false, false, EPI>), grid, block, 0, g.s, A, B, g.c, g.m, g.n, g.k, g.sa, g.sb, g.sc, g.up);
-    }
-    return launch_status("matmul (fp32 MFMA) launch");
+  if (mfma) {
+    const dim3 grid(((g.m + 255) / 256) * ((g.n + 255) / 256), g.batch);
+    return g.bt ? gemm_mfma_go<DT, DTO, EPI, true>(g, grid)
+                : gemm_mfma_go<DT, DTO, EPI, false>(g, grid);
   }
   const dim3 grid(((g.m + 63) / 64) * ((g.n + 63) / 64), g.batch), block(256);
   if (g.bt)
@@ -180,9 +141,10 @@ int gemm_launch(const GemmArgs& g, bool mfma) {
 
 template <int EPI>
 int gemm_dispatch(const GemmArgs& g, th_dtype in, th_dtype out) {
-  // f32 operands have no MFMA path; 16-bit ones need K % 8 == 0, row-major B
-  // N % 8 == 0 and 16-byte aligned operands and strides.
-  const bool mfma = in != TH_F32 && (g.k % 8 == 0) && (g.bt || g.n % 8 == 0) && aligned16(g.a) &&
+  if (in == TH_F32) return gemm_f32(g, out, EPI);
+  // the 16-bit MFMA paths need K % 8 == 0, row-major B N % 8 == 0 and 16-byte aligned
+  // operands and strides
+  const bool mfma = (g.k % 8 == 0) && (g.bt || g.n % 8 == 0) && aligned16(g.a) &&
                     aligned16(g.b) && (g.sa % 8 == 0) && (g.sb % 8 == 0);
   auto by_out = [&](auto dt) {
     constexpr int DT = decltype(dt)::value;
@@ -192,14 +154,37 @@ int gemm_dispatch(const GemmArgs& g, th_dtype in, th_dtype out) {
       default: return gemm_launch<DT, th::kBF16, EPI>(g, mfma);
     }
   };
-  switch (in) {
-    case TH_F32: return by_out(std::integral_constant<int, th::kF32>{});
-    case TH_F16: return by_out(std::integral_constant<int, th::kF16>{});
-    default: return by_out(std::integral_constant<int, th::kBF16>{});
-  }
+  if (in == TH_F16) return by_out(std::integral_constant<int, th::kF16>{});
+  return by_out(std::integral_constant<int, th::kBF16>{});
 }
 
 }  // namespace
+
+namespace th {
+namespace ops {
+
+int splitk_merge(const GemmArgs& g, const float* W, uint32_t S, th_dtype out, int epi) {
+  const uint64_t mn = static_cast<uint64_t>(g.m) * g.n;
+  const uint32_t blocks = static_cast<uint32_t>(
+      std::min<uint64_t>((mn + 255) / 256, 4ull * current_cu_count()));
+  auto go = [&](auto dto, auto e) {
+    hipLaunchKernelGGL((th::gemm_splitk_reduce<dto.value, e.value>), dim3(blocks), dim3(256), 0,
+                       g.s, W, g.c, g.up, mn, S);
+  };
+  auto by_epi = [&](auto dto) {
+    if (epi == th::gemm::kEpiSiluMul) go(dto, std::integral_constant<int, th::gemm::kEpiSiluMul>{});
+    else go(dto, std::integral_constant<int, th::gemm::kEpiStore>{});
+  };
+  switch (out) {
+    case TH_F32: by_epi(std::integral_constant<int, th::kF32>{}); break;
+    case TH_F16: by_epi(std::integral_constant<int, th::kF16>{}); break;
+    default: by_epi(std::integral_constant<int, th::kBF16>{}); break;
+  }
+  return launch_status("matmul (split-K merge) launch");
+}
+
+}  // namespace ops
+}  // namespace th
 
 extern "C" {
 

@@ -1,0 +1,34 @@
+// Shared by the GEMM translation units (ops_gemm.hip: entry points and 16-bit operands;
+// ops_gemm_f32.hip: f32 operands).
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+#include "ops_common.hpp"
+
+namespace th {
+namespace ops {
+
+// One GEMM launch: C[i] = epilogue(A[i] . B[i]) for i < batch, element strides
+// sa, sb, sc; `up` (epilogue kEpiSiluMul) has C's dtype, layout and strides.
+struct GemmArgs {
+  const void* a;
+  const void* b;
+  void* c;
+  const void* up;
+  uint32_t m, k, n;
+  bool bt;
+  uint32_t batch;
+  uint64_t sa, sb, sc;
+  hipStream_t s;
+};
+
+// C = epilogue(sum of the S partials of M x N f32 at W, in ascending order).
+int splitk_merge(const GemmArgs& g, const float* W, uint32_t S, th_dtype out, int epi);
+
+// f32 operands.
+int gemm_f32(const GemmArgs& g, th_dtype out, int epi);
+
+}  // namespace ops
+}  // namespace th
