@@ -69,9 +69,9 @@ __device__ __forceinline__ int swz(int row, int chunk) {
 template <int GM = GROUP_M>
 __device__ __forceinline__ void tile_coords(uint32_t bid, uint32_t tiles_m, uint32_t tiles_n,
                                             uint32_t& tm, uint32_t& tn) {
-  const uint32_t total = tiles_m * tiles_n;
-  uint32_t id = bid;
-  if (total % NXCD == 0) id = (bid % NXCD) * (total / NXCD) + bid / NXCD;
+  // each XCD (bid % NXCD) takes a contiguous run of ids, the first total % NXCD one more
+  const uint32_t total = tiles_m * tiles_n, x = bid % NXCD;
+  const uint32_t id = x * (total / NXCD) + min(x, total % NXCD) + bid / NXCD;
   const uint32_t per_group = GM * tiles_n;
   const uint32_t group = id / per_group;
   const uint32_t first_m = group * GM;

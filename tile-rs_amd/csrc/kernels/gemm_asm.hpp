@@ -1,6 +1,8 @@
-// Dense 16-bit GEMM on whole 256 x 256 tiles: the library's kernel for M and N multiples
-// of 256 and K a multiple of 128 (at least 256), B row-major (K x N) or stored N x K
-// (BT, __tile_matmul_transposed_f16: crates/tile_std/src/tile.rs:2028).
+// Dense 16-bit GEMM on whole 256 x 256 tiles: the library's kernel for M and N of at least
+// 256 and K a multiple of 128 (at least 256), B row-major (K x N) or stored N x K
+// (BT, __tile_matmul_transposed_f16: crates/tile_std/src/tile.rs:2028).  Where 256 does not
+// divide M (or N) the last tile row (column) starts at M - 256: it recomputes rows of the
+// one before it, the same bits from the same K order, so there is no edge code at all.
 //
 // The tile program is generated gfx950 assembly (gen_gemm.py, run by the build into
 // kernels/gen/gemm_asm.inc): four waves of 128 x 128 with AGPR accumulators
@@ -19,15 +21,17 @@
 namespace th {
 namespace gasm {
 constexpr int NT = 256;   // 4 waves
-// Shapes the program takes: whole tiles, K in groups of four 32-deep steps (at least
-// two groups), and every per-lane byte offset within 32 bits.
+// Shapes the kernel takes: at least one whole tile each way, K in groups of four 32-deep
+// steps (at least two groups), and every per-lane byte offset within 32 bits.  A ragged N
+// also needs every tile column to start on 16 bytes of a row-major B (and of UP): N % 8.
 __host__ __device__ constexpr bool fits(uint64_t m, uint64_t n, uint64_t k, int out_size) {
-  return m % 256 == 0 && n % 256 == 0 && k % 128 == 0 && k >= 256 && m > 0 && n > 0 &&
-         256 * k * 2 < (1ull << 31) && 136 * n * out_size < (1ull << 31) && 32 * n * 2 < (1ull << 31);
+  return m >= 256 && n >= 256 && k % 128 == 0 && k >= 256 && 256 * k * 2 < (1ull << 31) &&
+         136 * n * out_size < (1ull << 31) && 32 * n * 2 < (1ull << 31);
 }
 }  // namespace gasm
 
-// Tile (tm, tn) of C = A . B by a workgroup of gasm::NT threads (launched with at most
+// The 256 x 256 tile at row 256 tm, column 256 tn (or the last 256 rows, columns) of C =
+// A . B by a workgroup of gasm::NT threads (launched with at most
 // one workgroup per CU: the program uses all 512 registers of each lane).  A, B
 // 16-byte aligned, C aligned to its element; gasm::fits(M, N, K, sizeof C) holds.  A
 // workgroup that runs several tiles passes a barrier between them (the next tile's
@@ -47,7 +51,7 @@ __device__ __forceinline__ void gemm_asm_tile(const uint16_t* __restrict__ A,
   u32x4* arena = lds::dma_lds_arena<131072>();
   typedef __attribute__((address_space(3))) const void* lds_cptr;
   const uint32_t lds = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_cptr)(arena)));
-  const uint32_t m0 = tm * 256, n0 = tn * 256;
+  const uint32_t m0 = min(tm * 256, M - 256), n0 = min(tn * 256, N - 256);
   const uint32_t lane = threadIdx.x & 63;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t wm = wave >> 1, wn = wave & 1;
@@ -188,7 +192,7 @@ gemm_asm_256(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, voi
              const void* __restrict__ UP = nullptr) {
   constexpr uint32_t OSZ = (DT_OUT == kF32) ? 4 : 2;
   uint32_t tm, tn;
-  gemm::tile_coords(blockIdx.x, M / 256, N / 256, tm, tn);
+  gemm::tile_coords(blockIdx.x, (M + 255) / 256, (N + 255) / 256, tm, tn);
   const size_t coff = static_cast<size_t>(blockIdx.y) * sc * OSZ;
   gemm_asm_tile<DT, DT_OUT, BT, SILU>(A + blockIdx.y * sa, B + blockIdx.y * sb,
                                       static_cast<char*>(C) + coff, M, N, K, tm, tn,
