@@ -158,6 +158,7 @@ int gemm_dispatch(const GemmArgs& g, th_dtype in, th_dtype out) {
   // operands and strides
   const bool mfma = (g.k % 8 == 0) && (g.bt || g.n % 8 == 0) && aligned16(g.a) &&
                     aligned16(g.b) && (g.sa % 8 == 0) && (g.sb % 8 == 0);
+  if (mfma && few_rows_fit(g)) return gemm_few_rows(g, in, out, EPI);
   auto by_out = [&](auto dt) {
     constexpr int DT = decltype(dt)::value;
     switch (out) {

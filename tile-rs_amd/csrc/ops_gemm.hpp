@@ -1,5 +1,5 @@
 // Shared by the GEMM translation units (ops_gemm.hip: entry points and 16-bit operands;
-// ops_gemm_f32.hip: f32 operands).
+// ops_gemm_skinny.hip: 16-bit operands with few rows; ops_gemm_f32.hip: f32 operands).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -29,6 +29,11 @@ int splitk_merge(const GemmArgs& g, const float* W, uint32_t S, th_dtype out, in
 
 // f32 operands.
 int gemm_f32(const GemmArgs& g, th_dtype out, int epi);
+
+// 16-bit operands, few rows of A, B stored N x K: whether the kernel is the one for the
+// shape, and its launch (K % 8 == 0, A and B and their strides 16-byte aligned).
+bool few_rows_fit(const GemmArgs& g);
+int gemm_few_rows(const GemmArgs& g, th_dtype in, th_dtype out, int epi);
 
 }  // namespace ops
 }  // namespace th
