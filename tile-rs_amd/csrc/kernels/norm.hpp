@@ -214,4 +214,40 @@ rms_norm_part_apply(const void* x, void* y, const float* __restrict__ st, uint32
   }
 }
 
+// A workgroup per row with the row in registers (roww::Row); arguments as
+// softmax_rows_wide.
+template <int DT, int NT, int NV>
+__global__ void __launch_bounds__(NT)
+rms_norm_rows_wide(const void* x, void* y, uint32_t cols, float eps) {
+  using R = roww::Row<DT, NT, NV>;
+  constexpr int E = R::E, NW = NT / 64;
+  const size_t off = static_cast<size_t>(blockIdx.x) * cols * R::ESZ;
+  char* yr = static_cast<char*>(y) + off;
+  R r;
+  r.load(static_cast<const char*>(x) + off, cols);
+  float ss = r.ex * r.ex;
+  r.each([&](int i) {
+    float f[E];
+    unpack16<DT>(r.v[i], f);
+#pragma unroll
+    for (int e = 0; e < E; ++e) ss = __builtin_fmaf(f[e], f[e], ss);
+  });
+  ss = wave_sum(ss);
+  if constexpr (NW > 1) {
+    __shared__ float red[NW];
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    ss = roww::total(red);
+  }
+  const float rs = 1.0f / __builtin_sqrtf(ss * (1.0f / static_cast<float>(cols)) + eps);
+  if (r.col < cols) st_elem<DT>(yr, r.col, r.ex * rs);
+  r.each([&](int i) {
+    float f[E];
+    unpack16<DT>(r.v[i], f);
+#pragma unroll
+    for (int e = 0; e < E; ++e) f[e] *= rs;
+    r.store(yr, i, f);
+  });
+}
+
 }  // namespace th

@@ -482,4 +482,133 @@ softmax_part_apply(const void* x, void* y, const float2* __restrict__ st, uint32
   }
 }
 
+// ---- a row per workgroup, any length up to 16384 vectors, any alignment ------------
+// The whole row in the registers of one workgroup (NT threads, NV 16-byte vectors each): one
+// read and one write of the row and one launch, where the chunk kernels above read it twice
+// in two.  The columns before the first 16-byte boundary and after the last whole vector
+// (fewer than a vector each) are held one per thread.  Bound: HBM with at least a row per
+// CU, else the one row's own exponentials and latency; row_wg_pays in ops.hip weighs it.
+//
+// Measured on MI355X against the chunk kernels: softmax 256 x 50257 f32 33.9 -> 20.9 us,
+// 1024 x 50257 f32 125 -> 84 (4.9 TB/s), 4096 x 1030 f32 19.4 -> 9.8; RMSNorm 8 x 16384 bf16
+// 6.9 -> 4.3, 4096 x 4100 bf16 22.8 -> 13.5.
+namespace roww {
+constexpr int kNT = 1024;
+constexpr uint32_t kMaxVec = kNT * 16;
+
+template <int DT, int NT, int NV>
+struct Row {
+  static constexpr int ESZ = (DT == kF32) ? 4 : 2;
+  static constexpr int E = Vec16<DT>::kElems;
+  u32x4 v[NV];
+  float ex;            // this thread's single column, if any
+  uint32_t nv, col;    // whole vectors; column of ex (or cols)
+  size_t mid;          // byte offset of the first vector
+
+  __device__ __forceinline__ void load(const char* row, uint32_t cols) {
+    const uint32_t t = threadIdx.x;
+    const uint32_t head = min(
+        cols, static_cast<uint32_t>((16u - (reinterpret_cast<uintptr_t>(row) & 15u)) & 15u) / ESZ);
+    nv = (cols - head) / E;
+    mid = static_cast<size_t>(head) * ESZ;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const uint32_t vi = static_cast<uint32_t>(i) * NT + t;
+      if (vi < nv) v[i] = ldg128_nt(row + mid + static_cast<size_t>(vi) * 16);
+    }
+    // the head on threads 0..6, the tail on threads 8..14
+    const uint32_t tail = head + nv * E + (t - 8);
+    col = t < head ? t : t >= 8 && tail < cols ? tail : cols;
+    ex = 0.0f;
+    if (col < cols) ex = ld_elem<DT>(row, col);
+  }
+  // f(i) for each vector i this thread has
+  template <class F>
+  __device__ __forceinline__ void each(F&& f) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+      if (static_cast<uint32_t>(i) * NT + threadIdx.x < nv) f(i);
+  }
+  __device__ __forceinline__ void store(char* row, int i, const float (&f)[E]) const {
+    stg128_nt(row + mid + (static_cast<size_t>(i) * NT + threadIdx.x) * 16, pack16<DT>(f));
+  }
+};
+
+// The waves' sums, added in 64 bits: a row's few last additions would otherwise make up most
+// of the error that all its values share (RMSNorm 256 x 50257 f32: 6.1e-8 against 5.5e-8 of
+// the chunk kernels).
+template <int NW>
+__device__ __forceinline__ float total(const float (&part)[NW]) {
+  double s = part[0];
+#pragma unroll
+  for (int w = 1; w < NW; ++w) s += part[w];
+  return static_cast<float>(s);
+}
+}  // namespace roww
+
+// Grid: a workgroup per row; x and y at the same 16-byte phase (they may be one buffer).
+// Maximum, then sum, over the workgroup, as in the other register kernels (a row of -inf
+// only gives NaN); f32 values are replaced by their exponentials in place, 16-bit ones take
+// them again for the output.
+template <int DT, int NT, int NV>
+__global__ void __launch_bounds__(NT)
+softmax_rows_wide(const void* x, void* y, uint32_t cols) {
+  using R = roww::Row<DT, NT, NV>;
+  constexpr int E = R::E, NW = NT / 64;
+  __shared__ float red[2][NW];
+  const int wave = threadIdx.x >> 6;
+  const bool first = (threadIdx.x & 63) == 0;
+  const size_t off = static_cast<size_t>(blockIdx.x) * cols * R::ESZ;
+  char* yr = static_cast<char*>(y) + off;
+  R r;
+  r.load(static_cast<const char*>(x) + off, cols);
+  const bool one = r.col < cols;
+  float m = one ? r.ex : -INFINITY, s = 0.0f;
+  r.each([&](int i) {
+    float f[E];
+    unpack16<DT>(r.v[i], f);
+#pragma unroll
+    for (int e = 0; e < E; ++e) m = fmaxf(m, f[e]);
+  });
+  m = wave_max(m);
+  if constexpr (NW > 1) {
+    if (first) red[0][wave] = m;
+    __syncthreads();
+    m = red[0][0];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) m = fmaxf(m, red[0][w]);
+  }
+  const float mb = m * kLog2e;
+  if (one) {
+    r.ex = exp2_fast(__builtin_fmaf(r.ex, kLog2e, -mb));
+    s = r.ex;
+  }
+  r.each([&](int i) {
+    float f[E];
+    unpack16<DT>(r.v[i], f);
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      f[e] = exp2_fast(__builtin_fmaf(f[e], kLog2e, -mb));
+      s += f[e];
+    }
+    if constexpr (DT == kF32) r.v[i] = pack16<DT>(f);
+  });
+  s = wave_sum(s);
+  if constexpr (NW > 1) {
+    if (first) red[1][wave] = s;
+    __syncthreads();
+    s = roww::total(red[1]);
+  }
+  const float inv = 1.0f / s;
+  if (one) st_elem<DT>(yr, r.col, r.ex * inv);
+  r.each([&](int i) {
+    float f[E];
+    unpack16<DT>(r.v[i], f);
+#pragma unroll
+    for (int e = 0; e < E; ++e)
+      f[e] = (DT == kF32 ? f[e] : exp2_fast(__builtin_fmaf(f[e], kLog2e, -mb))) * inv;
+    r.store(yr, i, f);
+  });
+}
+
 }  // namespace th

@@ -63,6 +63,37 @@ int softmax_long(const void* x, void* y, uint32_t rows, uint32_t cols, hipStream
   return launch_status("softmax launch");
 }
 
+// Rows that the aligned register kernels do not take: whether a workgroup per row (one
+// launch, the row read once) beats the chunk kernels.  Measured on MI355X: the former takes
+// 4.3 us and `ps` picoseconds per column of a CU's row (16-bit softmax 120, f32 softmax 100,
+// 16-bit RMSNorm 85, f32 65) for each row a CU runs in turn, or the bytes' time; the latter
+// 6.7 us and the bytes read and written at 4 TB/s.  E.g. softmax 256 x 50257 f32 21.4 us
+// against 34.0, 64 x 50257 10.9 against 15.7, but 8 x 50257 8.4 against 7.3; 64 x 128256
+// bf16 20.9 against 18.3.
+bool row_wg_pays(uint32_t rows, uint32_t cols, int esz, uint32_t ps, const void* x,
+                 const void* y) {
+  const uint64_t bytes = static_cast<uint64_t>(cols) * esz, cus = current_cu_count();
+  if ((bytes + 15) / 16 > th::roww::kMaxVec || rows > 0x7fffffffu || !same_phase16(x, y))
+    return false;
+  const uint64_t rounds = (rows + cus - 1) / cus;
+  return rounds * cols * ps <= 2400000 + 2 * rows * bytes * 1000 / 4000;   // picoseconds
+}
+
+// The row-per-workgroup kernel's size: launch(threads, vectors per thread).
+template <class F>
+void row_wg_by_size(uint32_t cols, int esz, F&& launch) {
+  const uint32_t vec = (cols * static_cast<uint32_t>(esz) + 15) / 16;
+  auto go = [&](auto nt, auto nv) { launch(nt, nv); };
+  using std::integral_constant;
+  if (vec <= 64 * 4) go(integral_constant<int, 64>{}, integral_constant<int, 4>{});
+  else if (vec <= 256 * 4) go(integral_constant<int, 256>{}, integral_constant<int, 4>{});
+  else if (vec <= 1024 * 2) go(integral_constant<int, 1024>{}, integral_constant<int, 2>{});
+  else if (vec <= 1024 * 4) go(integral_constant<int, 1024>{}, integral_constant<int, 4>{});
+  else if (vec <= 1024 * 8) go(integral_constant<int, 1024>{}, integral_constant<int, 8>{});
+  else if (vec <= 1024 * 13) go(integral_constant<int, 1024>{}, integral_constant<int, 13>{});
+  else go(integral_constant<int, 1024>{}, integral_constant<int, 16>{});
+}
+
 template <int DT>
 int softmax_launch(const void* x, void* y, uint32_t rows, uint32_t cols, hipStream_t s) {
   constexpr int E = th::Vec16<DT>::kElems;
@@ -111,6 +142,11 @@ int softmax_launch(const void* x, void* y, uint32_t rows, uint32_t cols, hipStre
       hipLaunchKernelGGL((th::softmax_rows_reg<DT, 8>), grid, block, 0, s, x, y, rows, cols);
     else
       hipLaunchKernelGGL((th::softmax_rows_reg<DT, 16>), grid, block, 0, s, x, y, rows, cols);
+  } else if (row_wg_pays(rows, cols, 16 / E, E == 4 ? 100 : 120, x, y)) {
+    row_wg_by_size(cols, 16 / E, [&](auto nt, auto nv) {
+      hipLaunchKernelGGL((th::softmax_rows_wide<DT, nt.value, nv.value>), dim3(rows),
+                         dim3(nt.value), 0, s, x, y, cols);
+    });
   } else {
     return softmax_long<DT>(x, y, rows, cols, s);
   }
@@ -159,6 +195,11 @@ int rms_norm_launch(const void* x, void* y, uint32_t rows, uint32_t cols, float 
     else
       hipLaunchKernelGGL((th::rms_norm_rows_wg<DT, 16>), dim3(rows), dim3(256), 0, s, x, y, rows,
                          cols, eps);
+  } else if (row_wg_pays(rows, cols, 16 / E, E == 4 ? 65 : 85, x, y)) {
+    row_wg_by_size(cols, 16 / E, [&](auto nt, auto nv) {
+      hipLaunchKernelGGL((th::rms_norm_rows_wide<DT, nt.value, nv.value>), dim3(rows),
+                         dim3(nt.value), 0, s, x, y, cols, eps);
+    });
   } else {
     // long, ragged or unaligned rows: chunk sums of squares, then scale (as softmax_long)
     const uint64_t target = 4ull * current_cu_count();
