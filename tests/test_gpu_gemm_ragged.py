@@ -37,14 +37,13 @@ def both(call, c, stream):
     return out
 
 
-# K below 512 (or many tiles) keeps split K out of both runs
+# enough 256 x 256 tiles, and little enough K, that neither run takes smaller tiles or splits K
 @pytest.mark.parametrize("m,k,n,ind,outd,bt,bsz", [
-    (257, 256, 256, D.BF16, D.F32, False, 1),    # one row over: 255 rows recomputed
-    (511, 384, 264, D.F16, D.F16, False, 1),     # one short of whole; eight columns over
-    (256, 256, 504, D.BF16, D.BF16, False, 2),   # ragged N only, a batch
-    (300, 256, 300, D.F16, D.F32, True, 1),      # B stored N x K: N not a multiple of 8
-    (513, 384, 257, D.BF16, D.F16, True, 3),     # odd N: rows of C on odd 2-byte offsets
-    (3000, 512, 3008, D.BF16, D.F32, False, 1),  # 144 tiles
+    (3841, 256, 4096, D.BF16, D.F32, False, 1),   # one row over: 255 rows recomputed
+    (4095, 384, 3848, D.F16, D.F16, False, 1),    # one short of whole; eight columns over
+    (2048, 256, 4088, D.BF16, D.BF16, False, 2),  # ragged N only, a batch
+    (3900, 256, 3900, D.F16, D.F32, True, 1),     # B stored N x K: N not a multiple of 8
+    (1281, 384, 3999, D.BF16, D.F16, True, 3),    # odd N: rows of C on odd 2-byte offsets
 ])
 def test_ragged_matmul_same_bits_as_dma_kernel(dev, stream, m, k, n, ind, outd, bt, bsz):
     a = fill(dev, stream, bsz * m * k, ind, 1.0, 0x51)
@@ -55,8 +54,26 @@ def test_ragged_matmul_same_bits_as_dma_kernel(dev, stream, m, k, n, ind, outd, 
     assert np.array_equal(got, ref)   # the guard after C among it
 
 
+@pytest.mark.parametrize("ind", [D.BF16, D.F16])
+@pytest.mark.parametrize("outd", [D.BF16, D.F16])
+@pytest.mark.parametrize("bt", [False, True])
+def test_ragged_silu_mul_close_to_dma_kernel(dev, stream, ind, outd, bt):
+    """Every variant of the fused program, whole and overlapping tiles, against the LDS-DMA
+    kernel's expf and division: the GEMM tolerance."""
+    m, k, n = 4000, 256, 3848
+    a = fill(dev, stream, m * k, ind, 1.0, 0x71)
+    b = fill(dev, stream, k * n, ind, 0.2, 0x72)
+    up = fill(dev, stream, m * n, outd, 1.0, 0x73)
+    c = dev.alloc(m * n, outd)
+    got, ref = both(lambda: th.matmul_silu_mul(a, b, up, c, m, k, n, ind, outd, bt, stream=stream),
+                    c, stream)
+    assert_gemm_close(orc.widen(got, ORC[outd]), orc.widen(ref, ORC[outd]), "silu_mul",
+                      u16_dtype=ORC[outd])
+
+
 @pytest.mark.parametrize("in_place", [False, True])
-@pytest.mark.parametrize("m,k,n,dt,bt", [(300, 256, 264, D.F16, False), (513, 384, 256, D.BF16, True)])
+@pytest.mark.parametrize("m,k,n,dt,bt", [(3900, 256, 3848, D.F16, False),
+                                         (4000, 256, 3848, D.BF16, True)])
 def test_ragged_silu_mul(dev, stream, in_place, m, k, n, dt, bt):
     """Tiles that overlap must not read what another wrote where UP and C are one buffer."""
     a = fill(dev, stream, m * k, dt, 1.0, 0x61)
@@ -65,7 +82,8 @@ def test_ragged_silu_mul(dev, stream, in_place, m, k, n, dt, bt):
     up_host = up.copy_to_host(stream)
     c = up if in_place else dev.alloc(m * n, dt)
     th.matmul_silu_mul(a, b, up, c, m, k, n, dt, dt, bt, stream=stream)
+    got = orc.widen(c.copy_to_host(stream), ORC[dt]).reshape(m, n)[-300:]
     ref = orc.matmul_silu_mul(a.copy_to_host(stream), b.copy_to_host(stream), up_host, m, k, n,
-                              ORC[dt], ORC[dt], b_trans=bt)
-    assert_gemm_close(orc.widen(c.copy_to_host(stream), ORC[dt]), orc.widen(ref.reshape(-1), ORC[dt]),
+                              ORC[dt], ORC[dt], b_trans=bt, row0=m - 300, nrows=300)
+    assert_gemm_close(got, orc.widen(ref.reshape(-1), ORC[dt]).reshape(300, n),
                       f"silu_mul in_place={in_place}", u16_dtype=ORC[dt])

@@ -21,7 +21,7 @@ namespace {
 
 // ---- matmul -------------------------------------------------------------------
 
-// The LDS-DMA pipeline serves every shape with K % 32 == 0 unless
+// The LDS-DMA pipeline takes every shape with K % 32 == 0 that stays on 256 x 256 tiles, unless
 // TILERS_HIP_GEMM_DMA=0 (a debugging switch: the register-staged kernel then
 // runs them too).
 bool gemm_dma() {
@@ -83,6 +83,14 @@ int gemm_splitk(const GemmArgs& g, uint32_t tiles, uint32_t S) {
                       DTO == th::kF32 ? TH_F32 : DTO == th::kF16 ? TH_F16 : TH_BF16, EPI);
 }
 
+// Whether the LDS-DMA pipeline takes the product (its SiLU*Mul epilogue writes C and reads UP
+// in 16-byte pieces).
+bool dma_fits(const GemmArgs& g, int epi, uint64_t osz) {
+  return gemm_dma() && g.k % th::gemm::DBK == 0 &&
+         (epi != th::gemm::kEpiSiluMul ||
+          (aligned16(g.c) && aligned16(g.up) && (g.sc * osz) % 16 == 0 && g.n % 8 == 0));
+}
+
 // Whether UP and C share memory.
 bool overlap(const GemmArgs& g, uint64_t osz) {
   const uint64_t n = ((g.batch - 1) * g.sc + static_cast<uint64_t>(g.m) * g.n) * osz;
@@ -94,13 +102,9 @@ template <int DT, int DTO, int EPI, bool BT>
 int gemm_mfma_go(const GemmArgs& g, dim3 grid) {
   auto A = static_cast<const uint16_t*>(g.a);
   auto B = static_cast<const uint16_t*>(g.b);
-  // The DMA kernel's SiLU*Mul epilogue writes C and reads UP in 16-byte pieces.
   constexpr uint64_t OSZ = (DTO == th::kF32) ? 4 : 2;
-  const bool out_vec = EPI != th::gemm::kEpiSiluMul ||
-                       (aligned16(g.c) && aligned16(g.up) && (g.sc * OSZ) % 16 == 0 && g.n % 8 == 0);
-  if (gemm_dma() && out_vec && g.k % th::gemm::DBK == 0) {
-    const uint32_t S = splitk_slices(g, grid.x);
-    if (S > 1) return gemm_splitk<DT, DTO, EPI, BT>(g, grid.x, S);
+  if (dma_fits(g, EPI, OSZ)) {
+    if (g.slices > 1) return gemm_splitk<DT, DTO, EPI, BT>(g, grid.x, g.slices);
     // Ragged M or N included (SiLU*Mul, 3000 x 4096 x 14336 f16: 288 us here, 352 us on the
     // LDS-DMA kernel)
     const bool fits = th::gasm::fits(g.m, g.n, g.k, static_cast<int>(OSZ)) && gemm_asm();
@@ -159,12 +163,25 @@ int gemm_dispatch(const GemmArgs& g, th_dtype in, th_dtype out) {
   const bool mfma = (g.k % 8 == 0) && (g.bt || g.n % 8 == 0) && aligned16(g.a) &&
                     aligned16(g.b) && (g.sa % 8 == 0) && (g.sb % 8 == 0);
   if (mfma && few_rows_fit(g)) return gemm_few_rows(g, in, out, EPI);
+  GemmArgs h = g;
+  if (mfma) {
+    const uint64_t osz = dtype_size(out);
+    GemmForms f{false, dma_fits(g, EPI, osz), 1};
+    if (f.dma) {
+      f.whole = th::gasm::fits(g.m, g.n, g.k, static_cast<int>(osz)) && gemm_asm() &&
+                (EPI == th::gemm::kEpiStore || out != TH_F32);
+      f.split = splitk_slices(g, ((g.m + 255) / 256) * ((g.n + 255) / 256));
+    }
+    const GemmPlan plan = plan_16bit(g, f);
+    if (plan.tile != GemmPlan::k256) return gemm_mid_tiles(g, in, out, EPI, plan);
+    h.slices = plan.slices;
+  }
   auto by_out = [&](auto dt) {
     constexpr int DT = decltype(dt)::value;
     switch (out) {
-      case TH_F32: return gemm_launch<DT, th::kF32, EPI>(g, mfma);
-      case TH_F16: return gemm_launch<DT, th::kF16, EPI>(g, mfma);
-      default: return gemm_launch<DT, th::kBF16, EPI>(g, mfma);
+      case TH_F32: return gemm_launch<DT, th::kF32, EPI>(h, mfma);
+      case TH_F16: return gemm_launch<DT, th::kF16, EPI>(h, mfma);
+      default: return gemm_launch<DT, th::kBF16, EPI>(h, mfma);
     }
   };
   if (in == TH_F16) return by_out(std::integral_constant<int, th::kF16>{});

@@ -39,7 +39,7 @@ DEVICE_FLAGS = [
 ]
 HOST_CXX_FLAGS = ["-O2", "-std=c++17", "-fPIC", "-Wall", "-Wextra"]
 
-HIP_SOURCES = ["ops.hip", "ops_gemm.hip", "ops_gemm_skinny.hip",
+HIP_SOURCES = ["ops.hip", "ops_gemm.hip", "ops_gemm_mid.hip", "ops_gemm_skinny.hip",
                "ops_gemm_f32.hip", "runtime.cpp"]
 CPP_SOURCES = ["target/mlir_parse.cpp", "target/emit_hip.cpp", "target/registry.cpp"]
 
