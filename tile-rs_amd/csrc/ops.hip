@@ -49,7 +49,8 @@ int softmax_long(const void* x, void* y, uint32_t rows, uint32_t cols, hipStream
   const uint64_t blocks = static_cast<uint64_t>(rows) * parts;
   if (blocks > 0x7fffffffu) return fail(TH_KERNEL_ERROR, "softmax: grid too large");
   void* stv = nullptr;
-  TH_TRY(th::stream_scratch(s, blocks * sizeof(float2), &stv));
+  th::ScratchHold hold;
+  TH_TRY(th::stream_scratch(s, blocks * sizeof(float2), &stv, &hold));
   auto* st = static_cast<float2*>(stv);
   const dim3 grid(static_cast<uint32_t>(blocks)), block(256);
   const uint32_t P = static_cast<uint32_t>(parts), Cn = static_cast<uint32_t>(chunk);
@@ -211,7 +212,8 @@ int rms_norm_launch(const void* x, void* y, uint32_t rows, uint32_t cols, float 
     const uint64_t blocks = static_cast<uint64_t>(rows) * parts;
     if (blocks > 0x7fffffffu) return fail(TH_KERNEL_ERROR, "rms_norm: grid too large");
     void* stv = nullptr;
-    TH_TRY(th::stream_scratch(s, blocks * sizeof(float), &stv));
+    th::ScratchHold hold;
+    TH_TRY(th::stream_scratch(s, blocks * sizeof(float), &stv, &hold));
     auto* st = static_cast<float*>(stv);
     const dim3 grid(static_cast<uint32_t>(blocks)), block(256);
     const uint32_t P = static_cast<uint32_t>(parts), Cn = static_cast<uint32_t>(chunk);
@@ -470,9 +472,10 @@ int th_attention_prefill(const void* q, const void* k, const void* v, void* o, u
     const uint64_t split_bytes =
         nsplit > 1 ? static_cast<uint64_t>(nsplit) * rows_q * th::pfa::part_rec(hd) * 4 : 0;
     float* part_ws = nullptr;
+    th::ScratchHold hold;
     if (split_bytes && !pad) {
       void* ws = nullptr;
-      TH_TRY(th::stream_scratch(as_stream(s), split_bytes, &ws));
+      TH_TRY(th::stream_scratch(as_stream(s), split_bytes, &ws, &hold));
       part_ws = static_cast<float*>(ws);
     }
     if (pad) {
@@ -483,7 +486,7 @@ int th_attention_prefill(const void* q, const void* k, const void* v, void* o, u
       constexpr uint64_t RB = th::pfa::D * 2;  // bytes of a padded row
       void* ws = nullptr;
       const uint64_t pad_bytes = (2 * rows_q + 2 * rows_kv) * RB;
-      TH_TRY(th::stream_scratch(as_stream(s), pad_bytes + split_bytes, &ws));
+      TH_TRY(th::stream_scratch(as_stream(s), pad_bytes + split_bytes, &ws, &hold));
       auto* base = static_cast<uint16_t*>(ws);
       if (split_bytes) part_ws = reinterpret_cast<float*>(static_cast<char*>(ws) + pad_bytes);
       uint16_t* Qp = base;
@@ -732,12 +735,13 @@ int th_attention_decode(const void* q, const void* k, const void* v, void* o, ui
   const void* K = k;
   const void* V = v;
   void* O = o;
+  th::ScratchHold hold;
   if (pad) {
     constexpr uint64_t RB = th::dec::D * 2;
     const uint64_t rows_q = static_cast<uint64_t>(batch) * num_heads;
     const uint64_t rows_kv = static_cast<uint64_t>(batch) * num_kv_heads * seq_len;
     void* pw = nullptr;
-    TH_TRY(th::stream_scratch(as_stream(s), (2 * rows_q + 2 * rows_kv) * RB, &pw));
+    TH_TRY(th::stream_scratch(as_stream(s), (2 * rows_q + 2 * rows_kv) * RB, &pw, &hold));
     auto* base = static_cast<uint16_t*>(pw);
     uint16_t* Qp = base;
     uint16_t* Op = Qp + rows_q * th::dec::D;
@@ -778,7 +782,7 @@ int th_attention_decode(const void* q, const void* k, const void* v, void* o, ui
     }
     if (!ws && n_split > 1 &&
         (stream_capturing(as_stream(s)) ||
-         th::stream_scratch(as_stream(s), n_split * rec, &ws) != TH_OK)) {
+         th::stream_scratch(as_stream(s), n_split * rec, &ws, &hold) != TH_OK)) {
       ws = nullptr;
       decode_split_cap(decode_chunks(seq_len), 1, &n_split, &cps);
     }

@@ -62,7 +62,8 @@ int gemm_splitk(const GemmArgs& g, uint32_t tiles, uint32_t S) {
   const uint32_t ks = g.k / S;
   const uint64_t mn = static_cast<uint64_t>(g.m) * g.n;
   void* wv = nullptr;
-  TH_TRY(th::stream_scratch(g.s, S * mn * sizeof(float), &wv));
+  th::ScratchHold hold;
+  TH_TRY(th::stream_scratch(g.s, S * mn * sizeof(float), &wv, &hold));
   auto* W = static_cast<float*>(wv);
   auto go = [&](auto mi) {
     constexpr int MI = decltype(mi)::value;

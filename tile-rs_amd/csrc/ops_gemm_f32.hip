@@ -20,7 +20,8 @@ namespace {
 // one per CU, 102 us), and a split adds the merge: about 4 us and the partials' bytes, written
 // and read at about 4 TB/s.  The S with the least sum is taken.  No split while a graph is
 // recorded (its replays could meet on the stream's scratch) or without memory for it.
-uint32_t f32_slices(const GemmArgs& g, uint32_t tiles, uint32_t* ks, void** ws) {
+uint32_t f32_slices(const GemmArgs& g, uint32_t tiles, uint32_t* ks, void** ws,
+                    ScratchHold* hold) {
   *ks = g.k;
   if (g.batch != 1) return 1;
   const double cus = current_cu_count(), mn = static_cast<double>(g.m) * g.n;
@@ -37,7 +38,8 @@ uint32_t f32_slices(const GemmArgs& g, uint32_t tiles, uint32_t* ks, void** ws) 
     }
   }
   if (best == 1 || stream_capturing(g.s) ||
-      th::stream_scratch(g.s, best * static_cast<uint64_t>(g.m) * g.n * sizeof(float), ws) != TH_OK)
+      th::stream_scratch(g.s, best * static_cast<uint64_t>(g.m) * g.n * sizeof(float), ws, hold) !=
+          TH_OK)
     return 1;
   *ks = ((g.k + best - 1) / best + 63) / 64 * 64;
   return best;
@@ -69,7 +71,8 @@ int go(const GemmArgs& g, th_dtype out) {
     const uint32_t t64 = ((g.m + gf32s::BM - 1) / gf32s::BM) * ((g.n + gf32s::BN - 1) / gf32s::BN);
     void* ws = nullptr;
     uint32_t ks = 0;
-    const uint32_t S = f32_slices(g, t64, &ks, &ws);
+    ScratchHold hold;
+    const uint32_t S = f32_slices(g, t64, &ks, &ws, &hold);
     const dim3 grid(t64, g.batch, S), block(gf32s::NT);
     if (S > 1) {
       by_form([&](auto bt, auto v) {

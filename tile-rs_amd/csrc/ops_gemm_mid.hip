@@ -40,12 +40,13 @@ int by_tile(const GemmArgs& g, void* c, const GemmPlan& p) {
 template <int DT, int EPI>
 int go(const GemmArgs& g, th_dtype out, GemmPlan p) {
   void* ws = nullptr;
+  ScratchHold hold;
   // no split while a graph is recorded (its replays could meet on the stream's scratch) or
   // without memory for the partials
   if (p.slices > 1 &&
       (stream_capturing(g.s) ||
-       th::stream_scratch(g.s, static_cast<uint64_t>(p.slices) * g.m * g.n * sizeof(float), &ws) !=
-           TH_OK)) {
+       th::stream_scratch(g.s, static_cast<uint64_t>(p.slices) * g.m * g.n * sizeof(float), &ws,
+                          &hold) != TH_OK)) {
     p.slices = 1;
     p.ks = g.k;
   }

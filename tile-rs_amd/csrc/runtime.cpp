@@ -42,7 +42,12 @@ struct StreamKeyHash {
     return std::hash<const void*>()(k.stream) ^ (static_cast<size_t>(k.dev) << 1);
   }
 };
-std::unordered_map<StreamKey, Scratch, StreamKeyHash> g_stream_scratch;
+struct StreamScratch {
+  std::recursive_mutex mu;
+  Scratch buf;
+  std::vector<void*> outgrown;   // together smaller than buf
+};
+std::unordered_map<StreamKey, StreamScratch, StreamKeyHash> g_stream_scratch;
 }  // namespace
 
 int fail(int code, const std::string& msg) {
@@ -87,22 +92,33 @@ int device_scratch(size_t bytes, void** out) {
   return TH_OK;
 }
 
-int stream_scratch(hipStream_t stream, size_t bytes, void** out) {
+int stream_scratch(hipStream_t stream, size_t bytes, void** out, ScratchHold* hold) {
   int dev = 0;
   TH_TRY(check_hip(hipGetDevice(&dev), "hipGetDevice", TH_DEVICE_ERROR));
-  std::lock_guard<std::mutex> lock(g_scratch_mu);
-  Scratch& s = g_stream_scratch[StreamKey{dev, stream}];
+  StreamScratch* entry;
+  {
+    std::lock_guard<std::mutex> lock(g_scratch_mu);
+    entry = &g_stream_scratch[StreamKey{dev, stream}];   // (stays where it is)
+  }
+  *hold = ScratchHold(entry->mu);
+  Scratch& s = entry->buf;
   if (s.bytes < bytes) {
-    const size_t old_bytes = s.bytes;
-    if (s.ptr) {
-      // earlier work on this stream may still read the old buffer
+    const size_t want = std::max(bytes, std::max(size_t(64) << 10, 2 * s.bytes));
+    void* p = nullptr;
+    if (hipMalloc(&p, want) != hipSuccess) {
+      // out of memory: give the outgrown buffers back, once nothing queued reads them
+      (void)hipGetLastError();
+      if (s.ptr) entry->outgrown.push_back(s.ptr);
+      s = Scratch{};
       TH_TRY(check_hip(hipStreamSynchronize(stream), "hipStreamSynchronize", TH_STREAM_ERROR));
-      TH_TRY(check_hip(hipFree(s.ptr), "hipFree", TH_MEMORY_ERROR));
-      s.ptr = nullptr;
-      s.bytes = 0;
+      while (!entry->outgrown.empty()) {
+        TH_TRY(check_hip(hipFree(entry->outgrown.back()), "hipFree", TH_MEMORY_ERROR));
+        entry->outgrown.pop_back();
+      }
+      TH_TRY(check_hip(hipMalloc(&p, want), "hipMalloc", TH_MEMORY_ERROR));
     }
-    size_t want = std::max(bytes, std::max(size_t(64) << 10, 2 * old_bytes));
-    TH_TRY(check_hip(hipMalloc(&s.ptr, want), "hipMalloc", TH_MEMORY_ERROR));
+    if (s.ptr) entry->outgrown.push_back(s.ptr);
+    s.ptr = p;
     s.bytes = want;
   }
   *out = s.ptr;

@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <mutex>
 #include <string>
 
 #include "../../include/tilers_hip.h"
@@ -30,9 +31,15 @@ int device_scratch(size_t bytes, void** out);
 
 // Per-(device, stream) scratch for entry points without a workspace argument:
 // work queued on one stream runs in order, so calls never share the buffer
-// concurrently.  At least `bytes` (grown on demand after draining that stream,
-// kept until process exit).
-int stream_scratch(hipStream_t stream, size_t bytes, void** out);
+// concurrently.  `hold` locks the buffer until it is destroyed: a caller keeps it until
+// everything that uses the buffer is queued, so that another thread's call on the same
+// stream queues its work before or after and not in between, and cannot grow the buffer
+// meanwhile.  At least `bytes`, grown on demand to at least twice the size and kept until
+// process exit.  A buffer that is outgrown stays allocated while memory lasts (all of them
+// together are smaller than the current one): queued work and graphs recorded earlier still
+// use it.
+using ScratchHold = std::unique_lock<std::recursive_mutex>;
+int stream_scratch(hipStream_t stream, size_t bytes, void** out, ScratchHold* hold);
 
 }  // namespace th
 
