@@ -73,3 +73,41 @@ def test_mid_tiles_silu_mul(dev, stream, dt, out, trans, m, k, n):
         assert_gemm_close(got, ref, "silu_mul")
     else:
         assert_gemm_close(orc.widen(got, ORC[out]), ref, "silu_mul", u16_dtype=ORC[out])
+
+
+@pytest.mark.parametrize("warm", [True, False])
+def test_mid_tiles_recorded(dev, warm):
+    """A split product recorded into a graph: split if the stream's scratch is there already,
+    unsplit if not (recording never allocates), the same bits on every replay."""
+    from ctypes import byref, c_size_t, c_void_p
+
+    hip, s = th.lib(), dev.create_stream()
+    m, k, n = 8, 4096, 1024
+    rng = np.random.default_rng(5)
+    a = rng.integers(-4, 5, (m, k)).astype(np.float32)
+    b = rng.integers(-4, 5, (k, n)).astype(np.float32)
+    ab, bb = (put(dev, s, orc.narrow(x.ravel(), orc.BF16), D.BF16) for x in (a, b))
+    zero = np.zeros(m * n, np.float32)
+    cb, other = put(dev, s, zero, D.F32), put(dev, s, zero, D.F32)
+
+    def call(c):
+        th.matmul(ab, bb, c, m, k, n, D.BF16, D.F32, stream=s)
+
+    if warm:
+        call(other)
+    s.synchronize()
+    graph, run = c_void_p(), c_void_p()
+    assert hip.hipStreamBeginCapture(c_void_p(s.handle), 1) == 0
+    call(cb)
+    assert hip.hipStreamEndCapture(c_void_p(s.handle), byref(graph)) == 0
+    assert hip.hipGraphInstantiate(byref(run), graph, None, None, c_size_t(0)) == 0
+    ref = (a.astype(np.float64) @ b).astype(np.float32).ravel()
+    for _ in range(4):
+        cb.copy_from_host(zero, s)
+        call(other)   # eager work through the same scratch
+        assert hip.hipGraphLaunch(run, c_void_p(s.handle)) == 0
+        call(other)
+        assert np.array_equal(cb.copy_to_host(s), ref)
+        assert np.array_equal(other.copy_to_host(s), ref)
+    s.synchronize()
+    assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0

@@ -41,6 +41,7 @@ struct GemmPlan {
   enum { k64x64, k128x64, k256 };
   int tile;
   uint32_t slices, ks;
+  bool in_graph;   // split while a graph is recorded as well
 };
 // What the 256 x 256 kernels can do with it: the assembly kernel (whole), the LDS-DMA kernel
 // (dma; else the register-staged one), and the K split of the latter (1: none).

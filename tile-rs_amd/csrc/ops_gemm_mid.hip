@@ -41,12 +41,14 @@ template <int DT, int EPI>
 int go(const GemmArgs& g, th_dtype out, GemmPlan p) {
   void* ws = nullptr;
   ScratchHold hold;
-  // no split while a graph is recorded (its replays could meet on the stream's scratch) or
-  // without memory for the partials
+  // No split without memory for the partials.  While a graph is recorded (nothing can be
+  // allocated, and its replays could meet on the stream's scratch): only in place of a split
+  // on 256 x 256 tiles, which shares that buffer too, and if it is large enough already.
+  // (Row-major B 8 x 14336 x 4096 needs it: 64 workgroups unsplit.)
+  const uint64_t bytes = static_cast<uint64_t>(p.slices) * g.m * g.n * sizeof(float);
   if (p.slices > 1 &&
-      (stream_capturing(g.s) ||
-       th::stream_scratch(g.s, static_cast<uint64_t>(p.slices) * g.m * g.n * sizeof(float), &ws,
-                          &hold) != TH_OK)) {
+      ((stream_capturing(g.s) && !(p.in_graph && th::stream_scratch_ready(g.s, bytes))) ||
+       th::stream_scratch(g.s, bytes, &ws, &hold) != TH_OK)) {
     p.slices = 1;
     p.ks = g.k;
   }
@@ -95,10 +97,11 @@ GemmPlan plan_16bit(const GemmArgs& g, const GemmForms& f) {
                                          : 91.0 * std::ceil(w);
     return 3.0 + per * kk / s + merge_us(s);
   };
-  GemmPlan best{GemmPlan::k256, 1, g.k};
+  const bool in_graph = f.split > 1;
+  GemmPlan best{GemmPlan::k256, 1, g.k, in_graph};
   double best_us = est256(1);
   if (f.split > 1 && est256(f.split) < best_us) {
-    best = {GemmPlan::k256, f.split, g.k / f.split};
+    best = {GemmPlan::k256, f.split, g.k / f.split, in_graph};
     best_us = est256(f.split);
   }
   for (int tile : {GemmPlan::k128x64, GemmPlan::k64x64}) {
@@ -115,7 +118,7 @@ GemmPlan plan_16bit(const GemmArgs& g, const GemmForms& f) {
       if (big_b) per *= tile == GemmPlan::k128x64 ? (w > 1 ? 1.2 : 1.08) : g.bt ? 1.2 : 1.4;
       const double us = std::max(3.0 + per * ks / 4096.0, in_bytes / 3e6) + merge_us(s);
       if (us < best_us) {
-        best = {tile, s, ks};
+        best = {tile, s, ks, in_graph};
         best_us = us;
       }
     }

@@ -92,6 +92,20 @@ int device_scratch(size_t bytes, void** out) {
   return TH_OK;
 }
 
+bool stream_scratch_ready(hipStream_t stream, size_t bytes) {
+  int dev = 0;
+  if (check_hip(hipGetDevice(&dev), "hipGetDevice", TH_DEVICE_ERROR) != TH_OK) return false;
+  StreamScratch* entry;
+  {
+    std::lock_guard<std::mutex> lock(g_scratch_mu);
+    const auto it = g_stream_scratch.find(StreamKey{dev, stream});
+    if (it == g_stream_scratch.end()) return false;
+    entry = &it->second;
+  }
+  std::lock_guard<std::recursive_mutex> lock(entry->mu);
+  return entry->buf.bytes >= bytes;
+}
+
 int stream_scratch(hipStream_t stream, size_t bytes, void** out, ScratchHold* hold) {
   int dev = 0;
   TH_TRY(check_hip(hipGetDevice(&dev), "hipGetDevice", TH_DEVICE_ERROR));

@@ -41,6 +41,9 @@ int device_scratch(size_t bytes, void** out);
 using ScratchHold = std::unique_lock<std::recursive_mutex>;
 int stream_scratch(hipStream_t stream, size_t bytes, void** out, ScratchHold* hold);
 
+// Whether the stream's buffer holds `bytes` already, so that stream_scratch need not allocate.
+bool stream_scratch_ready(hipStream_t stream, size_t bytes);
+
 }  // namespace th
 
 #define TH_TRY(expr)                 \
