@@ -168,8 +168,8 @@ int th_matmul(const void* a, const void* b, void* c, uint32_t m, uint32_t k, uin
  * -> __tile_mul_* (tile.rs:229, :1135; linalg mlir_to_linalg.rs:449-451,
  * :774-782, :425; the gpu target fuses silu+mul the same way,
  * mlir_to_gpu.rs:536-634).  UP has out_dtype and C's layout and strides;
- * arithmetic is f32 with one rounding at the output (whole 256 x 256 tiles with
- * 16-bit C evaluate exp and the division with the hardware's f32 exp2 and
+ * arithmetic is f32 with one rounding at the output (the 256 x 256 assembly tiles
+ * with 16-bit C evaluate exp and the division with the hardware's f32 exp2 and
  * reciprocal, within the GEMM tolerance of the exact form).  Other arguments as
  * th_matmul. */
 int th_matmul_silu_mul(const void* a, const void* b, const void* up, void* c, uint32_t m,
@@ -208,6 +208,8 @@ int th_attention_prefill(const void* q, const void* k, const void* v, void* o, u
  * runtime params mlir_to_msl.rs:1816-1823 in the same order).
  * Q, O: [batch][num_heads][head_dim]; K, V: [batch][num_kv_heads][max_seq][head_dim];
  * positions [0, seq_len) are attended.
+ * f32 requires no workspace: it splits over the one given as far as that reaches,
+ * else over the stream's scratch.  For 16 bits
  * `workspace` may be NULL (the library keeps one per device, grown on demand;
  * calls that overlap on one device then race on it) or a device buffer of at
  * least th_attention_decode_workspace_size(...) bytes (non-zero for head_dim 128
