@@ -43,6 +43,8 @@ def inputs(rng, B, S, max_seq, Dh, NH, NKV):
     (1, 65, 64, 0, 4, 4),      # one query over, start on a stage edge
     (2, 300, 37, 3, 8, 8),     # 16 (batch, kv head) units on 8 XCDs: grouped work order
     (1, 257, 1000, 60, 4, 1),  # a chunk after cached positions, rows past it not read
+    (1, 601, 0, 0, 29, 29),    # 290 items: a short second round, not a multiple of 8
+    (4, 130, 0, 0, 56, 14),    # 672 items: a third round
 ])
 def test_prefill_f32_shapes(dev, stream, Dh, B, S, start, extra, NH, NKV):
     rng = np.random.default_rng(S * 7 + start + Dh)
