@@ -43,15 +43,7 @@ inline uint32_t current_cu_count() {
   return n;
 }
 
-// Whether work enqueued on `s` is being recorded into a graph.
-inline bool stream_capturing(hipStream_t s) {
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
-    (void)hipGetLastError();
-    return true;
-  }
-  return st != hipStreamCaptureStatusNone;
-}
+using th::stream_capturing;
 
 }  // namespace ops
 }  // namespace th

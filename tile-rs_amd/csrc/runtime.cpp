@@ -46,8 +46,56 @@ struct StreamScratch {
   std::recursive_mutex mu;
   Scratch buf;
   std::vector<void*> outgrown;   // together smaller than buf
+  bool recorded = false;         // handed out while a graph was recorded, which may use it later
 };
 std::unordered_map<StreamKey, StreamScratch, StreamKeyHash> g_stream_scratch;
+
+// hipStreamPerThread is one handle for a stream of its own in every thread, so there the
+// buffers belong to the thread (by device).  What ended threads leave is freed, a few of them
+// together, when a further thread asks for its first buffer there: hipFree waits for the device,
+// so nothing that they queued still runs.  What recorded graphs may use is never freed.
+constexpr size_t kLeftThreads = 16;
+using Left = std::unordered_map<int, std::vector<StreamScratch*>>;   // by device
+Left& left_by_threads() {   // (threads may end after static destructors)
+  static auto& v = *new Left;
+  return v;
+}
+struct ThreadScratch {
+  std::vector<std::pair<int, StreamScratch*>> own;
+  ~ThreadScratch() {
+    std::lock_guard<std::mutex> lock(g_scratch_mu);
+    for (const auto& e : own)
+      if (!e.second->recorded) left_by_threads()[e.first].push_back(e.second);
+  }
+};
+
+// The stream's entry (on device dev), or null if it has none and `make` is false; `recording`:
+// the stream is being captured, so nothing may be freed.
+StreamScratch* stream_entry(int dev, hipStream_t stream, bool make, bool recording = false) {
+  if (stream != hipStreamPerThread) {
+    std::lock_guard<std::mutex> lock(g_scratch_mu);
+    if (make) return &g_stream_scratch[StreamKey{dev, stream}];   // (stays where it is)
+    const auto it = g_stream_scratch.find(StreamKey{dev, stream});
+    return it == g_stream_scratch.end() ? nullptr : &it->second;
+  }
+  thread_local ThreadScratch mine;
+  for (const auto& e : mine.own)
+    if (e.first == dev) return e.second;
+  if (!make) return nullptr;
+  std::vector<StreamScratch*> old;
+  {
+    std::lock_guard<std::mutex> lock(g_scratch_mu);
+    auto& left = left_by_threads()[dev];
+    if (!recording && left.size() >= kLeftThreads) old.swap(left);
+  }
+  for (StreamScratch* e : old) {
+    for (void* p : e->outgrown) (void)hipFree(p);
+    if (e->buf.ptr) (void)hipFree(e->buf.ptr);
+    delete e;
+  }
+  mine.own.emplace_back(dev, new StreamScratch);
+  return mine.own.back().second;
+}
 }  // namespace
 
 int fail(int code, const std::string& msg) {
@@ -92,16 +140,20 @@ int device_scratch(size_t bytes, void** out) {
   return TH_OK;
 }
 
+bool stream_capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return st != hipStreamCaptureStatusNone;
+}
+
 bool stream_scratch_ready(hipStream_t stream, size_t bytes) {
   int dev = 0;
   if (check_hip(hipGetDevice(&dev), "hipGetDevice", TH_DEVICE_ERROR) != TH_OK) return false;
-  StreamScratch* entry;
-  {
-    std::lock_guard<std::mutex> lock(g_scratch_mu);
-    const auto it = g_stream_scratch.find(StreamKey{dev, stream});
-    if (it == g_stream_scratch.end()) return false;
-    entry = &it->second;
-  }
+  StreamScratch* entry = stream_entry(dev, stream, false);
+  if (!entry) return false;
   std::lock_guard<std::recursive_mutex> lock(entry->mu);
   return entry->buf.bytes >= bytes;
 }
@@ -109,12 +161,10 @@ bool stream_scratch_ready(hipStream_t stream, size_t bytes) {
 int stream_scratch(hipStream_t stream, size_t bytes, void** out, ScratchHold* hold) {
   int dev = 0;
   TH_TRY(check_hip(hipGetDevice(&dev), "hipGetDevice", TH_DEVICE_ERROR));
-  StreamScratch* entry;
-  {
-    std::lock_guard<std::mutex> lock(g_scratch_mu);
-    entry = &g_stream_scratch[StreamKey{dev, stream}];   // (stays where it is)
-  }
+  const bool recording = stream_capturing(stream);
+  StreamScratch* entry = stream_entry(dev, stream, true, recording);
   *hold = ScratchHold(entry->mu);
+  entry->recorded = entry->recorded || recording;
   Scratch& s = entry->buf;
   if (s.bytes < bytes) {
     const size_t want = std::max(bytes, std::max(size_t(64) << 10, 2 * s.bytes));

@@ -29,9 +29,14 @@ int use_device(int ordinal);
 // demand, kept until process exit).
 int device_scratch(size_t bytes, void** out);
 
+// Whether work enqueued on `s` is being recorded into a graph (or that cannot be told).
+bool stream_capturing(hipStream_t s);
+
 // Per-(device, stream) scratch for entry points without a workspace argument:
 // work queued on one stream runs in order, so calls never share the buffer
-// concurrently.  `hold` locks the buffer until it is destroyed: a caller keeps it until
+// concurrently.  (hipStreamPerThread names another stream in every thread: there each
+// thread has a buffer of its own, freed some time after the thread has ended unless a graph
+// recorded it.)  `hold` locks the buffer until it is destroyed: a caller keeps it until
 // everything that uses the buffer is queued, so that another thread's call on the same
 // stream queues its work before or after and not in between, and cannot grow the buffer
 // meanwhile.  At least `bytes`, grown on demand to at least twice the size and kept until
