@@ -116,12 +116,54 @@ void per_thread_bounded() {
   CHECK(g_live.count(graphs));
   CHECK(live_bytes() <= MB + 17 * 6 * MB);
 }
+
+// A graph recorded earlier uses its buffer whenever it is replayed: where memory runs out, that
+// buffer stays, as the current one or outgrown; others make room.
+void short_of_memory() {
+  get(kA, 2 * MB);
+  g_capturing.insert(kA);
+  void* graphs = get(kA, 2 * MB);
+  g_capturing.clear();
+  g_capacity = 10 * MB;
+  CHECK(!get(kA, 12 * MB));
+  CHECK(g_live.count(graphs) && get(kA, 2 * MB) == graphs);
+  CHECK(get(kA, 3 * MB));   // 4 MB
+  CHECK(!get(kA, 9 * MB));
+  CHECK(g_live.count(graphs) && live_bytes() == 2 * MB);
+  CHECK(get(kA, 8 * MB) && get(kA, 8 * MB) != graphs);
+}
+
+// A call that can do without gives nothing back.
+void short_of_memory_optional() {
+  void* p = get(kA, 2 * MB);
+  g_capacity = 10 * MB;
+  void* q = nullptr;
+  {
+    th::ScratchHold hold;
+    CHECK(!th::try_stream_scratch(kA, 9 * MB, &q, &hold));
+  }
+  CHECK(g_live.count(p) && get(kA, 2 * MB) == p);
+  CHECK(get(kA, 9 * MB));   // a call that cannot do without makes room
+}
+
+// A refused allocation is no lack of memory: the buffer stays.
+void refused_while_recording() {
+  void* p = get(kA, MB);
+  g_capturing.insert(kA);
+  CHECK(!get(kA, 5 * MB));
+  g_capturing.clear();
+  CHECK(get(kA, MB) == p && live_bytes() == MB);
+  CHECK(get(kA, 5 * MB) && live_bytes() == 6 * MB);
+}
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::map<std::string, void (*)()> all = {
       {"per_thread_own", per_thread_own},
       {"per_thread_bounded", per_thread_bounded},
+      {"short_of_memory", short_of_memory},
+      {"short_of_memory_optional", short_of_memory_optional},
+      {"refused_while_recording", refused_while_recording},
   };
   const auto it = argc == 2 ? all.find(argv[1]) : all.end();
   CHECK(it != all.end());

@@ -23,7 +23,9 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["per_thread_own", "per_thread_bounded"])
+@pytest.mark.parametrize("scenario", [
+    "per_thread_own", "per_thread_bounded", "short_of_memory", "short_of_memory_optional",
+    "refused_while_recording"])
 def test_scratch(program, scenario):
     out = subprocess.run([str(program), scenario], stdout=subprocess.PIPE,
                          stderr=subprocess.STDOUT, text=True, timeout=60)

@@ -782,7 +782,7 @@ int th_attention_decode(const void* q, const void* k, const void* v, void* o, ui
     }
     if (!ws && n_split > 1 &&
         (stream_capturing(as_stream(s)) ||
-         th::stream_scratch(as_stream(s), n_split * rec, &ws, &hold) != TH_OK)) {
+         !th::try_stream_scratch(as_stream(s), n_split * rec, &ws, &hold))) {
       ws = nullptr;
       decode_split_cap(decode_chunks(seq_len), 1, &n_split, &cps);
     }

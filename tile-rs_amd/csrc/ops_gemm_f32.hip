@@ -38,8 +38,8 @@ uint32_t f32_slices(const GemmArgs& g, uint32_t tiles, uint32_t* ks, void** ws,
     }
   }
   if (best == 1 || stream_capturing(g.s) ||
-      th::stream_scratch(g.s, best * static_cast<uint64_t>(g.m) * g.n * sizeof(float), ws, hold) !=
-          TH_OK)
+      !th::try_stream_scratch(g.s, best * static_cast<uint64_t>(g.m) * g.n * sizeof(float), ws,
+                              hold))
     return 1;
   *ks = ((g.k + best - 1) / best + 63) / 64 * 64;
   return best;

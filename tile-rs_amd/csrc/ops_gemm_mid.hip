@@ -48,7 +48,7 @@ int go(const GemmArgs& g, th_dtype out, GemmPlan p) {
   const uint64_t bytes = static_cast<uint64_t>(p.slices) * g.m * g.n * sizeof(float);
   if (p.slices > 1 &&
       ((stream_capturing(g.s) && !(p.in_graph && th::stream_scratch_ready(g.s, bytes))) ||
-       th::stream_scratch(g.s, bytes, &ws, &hold) != TH_OK)) {
+       !th::try_stream_scratch(g.s, bytes, &ws, &hold))) {
     p.slices = 1;
     p.ks = g.k;
   }

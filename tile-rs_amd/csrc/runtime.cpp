@@ -42,11 +42,18 @@ struct StreamKeyHash {
     return std::hash<const void*>()(k.stream) ^ (static_cast<size_t>(k.dev) << 1);
   }
 };
+struct StreamBuffer : Scratch {
+  bool recorded = false;   // handed out while a graph was recorded, which may use it later
+};
 struct StreamScratch {
   std::recursive_mutex mu;
-  Scratch buf;
-  std::vector<void*> outgrown;   // together smaller than buf
-  bool recorded = false;         // handed out while a graph was recorded, which may use it later
+  StreamBuffer buf;
+  std::vector<StreamBuffer> outgrown;   // together smaller than buf, unless memory ran out
+
+  bool recorded() const {
+    return buf.recorded || std::any_of(outgrown.begin(), outgrown.end(),
+                                       [](const StreamBuffer& b) { return b.recorded; });
+  }
 };
 std::unordered_map<StreamKey, StreamScratch, StreamKeyHash> g_stream_scratch;
 
@@ -65,7 +72,7 @@ struct ThreadScratch {
   ~ThreadScratch() {
     std::lock_guard<std::mutex> lock(g_scratch_mu);
     for (const auto& e : own)
-      if (!e.second->recorded) left_by_threads()[e.first].push_back(e.second);
+      if (!e.second->recorded()) left_by_threads()[e.first].push_back(e.second);
   }
 };
 
@@ -89,7 +96,7 @@ StreamScratch* stream_entry(int dev, hipStream_t stream, bool make, bool recordi
     if (!recording && left.size() >= kLeftThreads) old.swap(left);
   }
   for (StreamScratch* e : old) {
-    for (void* p : e->outgrown) (void)hipFree(p);
+    for (const StreamBuffer& b : e->outgrown) (void)hipFree(b.ptr);
     if (e->buf.ptr) (void)hipFree(e->buf.ptr);
     delete e;
   }
@@ -158,35 +165,56 @@ bool stream_scratch_ready(hipStream_t stream, size_t bytes) {
   return entry->buf.bytes >= bytes;
 }
 
-int stream_scratch(hipStream_t stream, size_t bytes, void** out, ScratchHold* hold) {
+namespace {
+// A buffer of at least `bytes` in place of the entry's.  Where memory is short and may_free, the
+// buffers that no recorded graph may use are given back first, once nothing queued reads them.
+// On failure the entry keeps every buffer that was not given back.
+int grow(StreamScratch& e, hipStream_t stream, size_t bytes, bool may_free) {
+  const size_t want = std::max(bytes, std::max(size_t(64) << 10, 2 * e.buf.bytes));
+  void* p = nullptr;
+  hipError_t err = hipMalloc(&p, want);
+  if (err == hipErrorOutOfMemory && may_free) {
+    (void)hipGetLastError();
+    TH_TRY(check_hip(hipStreamSynchronize(stream), "hipStreamSynchronize", TH_STREAM_ERROR));
+    for (size_t i = e.outgrown.size(); i-- > 0;) {
+      if (e.outgrown[i].recorded) continue;
+      TH_TRY(check_hip(hipFree(e.outgrown[i].ptr), "hipFree", TH_MEMORY_ERROR));
+      e.outgrown.erase(e.outgrown.begin() + static_cast<ptrdiff_t>(i));
+    }
+    if (e.buf.ptr && !e.buf.recorded) {
+      TH_TRY(check_hip(hipFree(e.buf.ptr), "hipFree", TH_MEMORY_ERROR));
+      e.buf = StreamBuffer{};
+    }
+    err = hipMalloc(&p, want);
+  }
+  TH_TRY(check_hip(err, "hipMalloc", TH_MEMORY_ERROR));
+  if (e.buf.ptr) e.outgrown.push_back(e.buf);
+  e.buf = StreamBuffer{};
+  e.buf.ptr = p;
+  e.buf.bytes = want;
+  return TH_OK;
+}
+
+int stream_buffer(hipStream_t stream, size_t bytes, bool may_free, void** out,
+                  ScratchHold* hold) {
   int dev = 0;
   TH_TRY(check_hip(hipGetDevice(&dev), "hipGetDevice", TH_DEVICE_ERROR));
   const bool recording = stream_capturing(stream);
   StreamScratch* entry = stream_entry(dev, stream, true, recording);
   *hold = ScratchHold(entry->mu);
-  entry->recorded = entry->recorded || recording;
-  Scratch& s = entry->buf;
-  if (s.bytes < bytes) {
-    const size_t want = std::max(bytes, std::max(size_t(64) << 10, 2 * s.bytes));
-    void* p = nullptr;
-    if (hipMalloc(&p, want) != hipSuccess) {
-      // out of memory: give the outgrown buffers back, once nothing queued reads them
-      (void)hipGetLastError();
-      if (s.ptr) entry->outgrown.push_back(s.ptr);
-      s = Scratch{};
-      TH_TRY(check_hip(hipStreamSynchronize(stream), "hipStreamSynchronize", TH_STREAM_ERROR));
-      while (!entry->outgrown.empty()) {
-        TH_TRY(check_hip(hipFree(entry->outgrown.back()), "hipFree", TH_MEMORY_ERROR));
-        entry->outgrown.pop_back();
-      }
-      TH_TRY(check_hip(hipMalloc(&p, want), "hipMalloc", TH_MEMORY_ERROR));
-    }
-    if (s.ptr) entry->outgrown.push_back(s.ptr);
-    s.ptr = p;
-    s.bytes = want;
-  }
-  *out = s.ptr;
+  if (entry->buf.bytes < bytes) TH_TRY(grow(*entry, stream, bytes, may_free && !recording));
+  entry->buf.recorded = entry->buf.recorded || recording;
+  *out = entry->buf.ptr;
   return TH_OK;
+}
+}  // namespace
+
+int stream_scratch(hipStream_t stream, size_t bytes, void** out, ScratchHold* hold) {
+  return stream_buffer(stream, bytes, true, out, hold);
+}
+
+bool try_stream_scratch(hipStream_t stream, size_t bytes, void** out, ScratchHold* hold) {
+  return stream_buffer(stream, bytes, false, out, hold) == TH_OK;
 }
 
 }  // namespace th

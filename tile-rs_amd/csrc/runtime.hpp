@@ -40,11 +40,16 @@ bool stream_capturing(hipStream_t s);
 // everything that uses the buffer is queued, so that another thread's call on the same
 // stream queues its work before or after and not in between, and cannot grow the buffer
 // meanwhile.  At least `bytes`, grown on demand to at least twice the size and kept until
-// process exit.  A buffer that is outgrown stays allocated while memory lasts (all of them
-// together are smaller than the current one): queued work and graphs recorded earlier still
-// use it.
+// process exit.  A buffer that is outgrown stays allocated (all of them together are smaller
+// than the current one): queued work and graphs recorded earlier still use it.  Only where
+// memory runs out are a stream's buffers given back to make room, after draining the stream,
+// but for those that were handed out while a graph was recorded.
 using ScratchHold = std::unique_lock<std::recursive_mutex>;
 int stream_scratch(hipStream_t stream, size_t bytes, void** out, ScratchHold* hold);
+
+// The same for a caller that can do without: false, and nothing given back, where the memory
+// for it cannot be had.
+bool try_stream_scratch(hipStream_t stream, size_t bytes, void** out, ScratchHold* hold);
 
 // Whether the stream's buffer holds `bytes` already, so that stream_scratch need not allocate.
 bool stream_scratch_ready(hipStream_t stream, size_t bytes);
