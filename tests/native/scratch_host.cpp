@@ -155,6 +155,20 @@ void refused_while_recording() {
   CHECK(get(kA, MB) == p && live_bytes() == MB);
   CHECK(get(kA, 5 * MB) && live_bytes() == 6 * MB);
 }
+
+// Another stream is being captured in global mode: allocations and frees here neither fail nor
+// break that capture, and the thread's own mode is as it was.
+void another_stream_recorded() {
+  const hipStream_t other = reinterpret_cast<hipStream_t>(0x2000);
+  for (int i = 0; i < 16; ++i) in_thread(hipStreamPerThread, MB);   // left to be freed
+  g_capturing.insert(other);
+  CHECK(get(kA, MB));
+  CHECK(get(kA, 3 * MB));
+  CHECK(in_thread(hipStreamPerThread, MB) && live_bytes() == 5 * MB);
+  g_capacity = 10 * MB;
+  CHECK(get(kA, 7 * MB));   // makes room
+  CHECK(g_invalidated == 0 && t_mode == hipStreamCaptureModeGlobal);
+}
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -164,6 +178,7 @@ int main(int argc, char** argv) {
       {"short_of_memory", short_of_memory},
       {"short_of_memory_optional", short_of_memory_optional},
       {"refused_while_recording", refused_while_recording},
+      {"another_stream_recorded", another_stream_recorded},
   };
   const auto it = argc == 2 ? all.find(argv[1]) : all.end();
   CHECK(it != all.end());

@@ -25,7 +25,7 @@ def program(tmp_path_factory):
 
 @pytest.mark.parametrize("scenario", [
     "per_thread_own", "per_thread_bounded", "short_of_memory", "short_of_memory_optional",
-    "refused_while_recording"])
+    "refused_while_recording", "another_stream_recorded"])
 def test_scratch(program, scenario):
     out = subprocess.run([str(program), scenario], stdout=subprocess.PIPE,
                          stderr=subprocess.STDOUT, text=True, timeout=60)

@@ -42,6 +42,27 @@ struct StreamKeyHash {
     return std::hash<const void*>()(k.stream) ^ (static_cast<size_t>(k.dev) << 1);
   }
 };
+// While any stream of the process is captured in global mode, hipMalloc and hipFree are refused
+// and break that capture, although this memory belongs to none.  So the calling thread's mode
+// is relaxed meanwhile (not for a call that is being captured itself: the caller's mode decides).
+class RelaxedCaptureMode {
+ public:
+  explicit RelaxedCaptureMode(bool relax) : relaxed_(relax) { exchange(); }
+  ~RelaxedCaptureMode() { exchange(); }
+  RelaxedCaptureMode(const RelaxedCaptureMode&) = delete;
+  RelaxedCaptureMode& operator=(const RelaxedCaptureMode&) = delete;
+
+ private:
+  void exchange() {
+    if (relaxed_ && hipThreadExchangeStreamCaptureMode(&mode_) != hipSuccess) {
+      (void)hipGetLastError();
+      relaxed_ = false;
+    }
+  }
+  bool relaxed_;
+  hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;   // then the thread's own
+};
+
 struct StreamBuffer : Scratch {
   bool recorded = false;   // handed out while a graph was recorded, which may use it later
 };
@@ -95,6 +116,7 @@ StreamScratch* stream_entry(int dev, hipStream_t stream, bool make, bool recordi
     auto& left = left_by_threads()[dev];
     if (!recording && left.size() >= kLeftThreads) old.swap(left);
   }
+  const RelaxedCaptureMode relaxed(!old.empty());
   for (StreamScratch* e : old) {
     for (const StreamBuffer& b : e->outgrown) (void)hipFree(b.ptr);
     if (e->buf.ptr) (void)hipFree(e->buf.ptr);
@@ -202,7 +224,10 @@ int stream_buffer(hipStream_t stream, size_t bytes, bool may_free, void** out,
   const bool recording = stream_capturing(stream);
   StreamScratch* entry = stream_entry(dev, stream, true, recording);
   *hold = ScratchHold(entry->mu);
-  if (entry->buf.bytes < bytes) TH_TRY(grow(*entry, stream, bytes, may_free && !recording));
+  if (entry->buf.bytes < bytes) {
+    const RelaxedCaptureMode relaxed(!recording);
+    TH_TRY(grow(*entry, stream, bytes, may_free && !recording));
+  }
   entry->buf.recorded = entry->buf.recorded || recording;
   *out = entry->buf.ptr;
   return TH_OK;
