@@ -22,7 +22,13 @@ CASES = [(4096, 512, 4096, D.BF16, D.F32, False), (2048, 1024, 4608, D.F16, D.F1
          (4096, 512, 2304, D.BF16, D.BF16, True)]
 
 
-@pytest.mark.parametrize("m,k,n,ind,outd,bt", CASES)
+# products that would be split over K, or run on smaller tiles, if the plan reckoned with the
+# LDS-DMA kernel's times: the switch changes the kernel alone
+PLAN_CASES = [(2048, 4096, 4096, D.BF16, D.F32, False), (4096, 4096, 2048, D.F16, D.F16, True),
+              (1792, 4096, 4096, D.BF16, D.BF16, False)]
+
+
+@pytest.mark.parametrize("m,k,n,ind,outd,bt", CASES + PLAN_CASES)
 def test_assembly_and_dma_kernels_agree_bitwise(dev, stream, m, k, n, ind, outd, bt):
     print(f"gemm paths {m}x{k}x{n} {ind}->{outd} bt={bt}", flush=True)
     a, b = dev.alloc(m * k, ind), dev.alloc(k * n, ind)

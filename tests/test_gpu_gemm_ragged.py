@@ -37,13 +37,15 @@ def both(call, c, stream):
     return out
 
 
-# enough 256 x 256 tiles, and little enough K, that neither run takes smaller tiles or splits K
+# enough 256 x 256 tiles, and little enough K, that smaller tiles or a split of K are estimated
+# longer (for all but the 1281-row product by half as much again)
 @pytest.mark.parametrize("m,k,n,ind,outd,bt,bsz", [
     (3841, 256, 4096, D.BF16, D.F32, False, 1),   # one row over: 255 rows recomputed
     (4095, 384, 3848, D.F16, D.F16, False, 1),    # one short of whole; eight columns over
     (2048, 256, 4088, D.BF16, D.BF16, False, 2),  # ragged N only, a batch
     (3900, 256, 3900, D.F16, D.F32, True, 1),     # B stored N x K: N not a multiple of 8
     (1281, 384, 3999, D.BF16, D.F16, True, 3),    # odd N: rows of C on odd 2-byte offsets
+    (1501, 384, 2497, D.BF16, D.F16, True, 4),    # odd N: rows of C on odd 2-byte offsets
 ])
 def test_ragged_matmul_same_bits_as_dma_kernel(dev, stream, m, k, n, ind, outd, bt, bsz):
     a = fill(dev, stream, bsz * m * k, ind, 1.0, 0x51)

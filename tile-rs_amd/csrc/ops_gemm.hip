@@ -169,7 +169,8 @@ int gemm_dispatch(const GemmArgs& g, th_dtype in, th_dtype out) {
     const uint64_t osz = dtype_size(out);
     GemmForms f{false, dma_fits(g, EPI, osz), 1};
     if (f.dma) {
-      f.whole = th::gasm::fits(g.m, g.n, g.k, static_cast<int>(osz)) && gemm_asm() &&
+      // (whatever TILERS_HIP_GEMM_ASM says: it swaps kernels on the same tiles and K split)
+      f.whole = th::gasm::fits(g.m, g.n, g.k, static_cast<int>(osz)) &&
                 (EPI == th::gemm::kEpiStore || out != TH_F32);
       f.split = splitk_slices(g, ((g.m + 255) / 256) * ((g.n + 255) / 256));
     }
