@@ -560,15 +560,19 @@ __device__ __forceinline__ void prefill_f32_tile(const float* __restrict__ Q,
   }
 }
 
-// Work index of workgroup w of `total`.  Two workgroups share each of the 256 CUs, and the
-// second to come runs beside the 256th before it: heavy first in both rounds would give one
-// CU the heaviest items of each.  So the second round runs light first (its XCD order kept): 1001
-// queries x 32 heads (512 items) 114.3 -> 92.9 us.
-__device__ __forceinline__ uint32_t prefill_f32_item(uint32_t w, uint32_t total) {
-  constexpr uint32_t kCus = 256;
-  if (w / kCus != 1) return w;
-  const uint32_t n = min(kCus, total - kCus), step = total % 8 == 0 ? 8 : 1, l = w - kCus;
-  return kCus + (n / step - 1 - l / step) * step + l % step;
+// Work index of workgroup w of `total` on a device of `cus` CUs.  The second workgroup of a CU
+// runs beside the one `cus` before it: heavy first in both rounds would give one CU the
+// heaviest items of each.  So the second round runs light first (its XCD order kept).
+// Measured on MI355X, 32 heads over 8, us with both rounds heavy first and now: 1001 queries
+// (512 items) 114.4 -> 91.7, D 64 63.4 -> 52.6; 640 (320) 64.5 -> 61.4; 1000 after 1024 250 ->
+// 225; later rounds stay heavy first: 1536 (768) 188 -> 190, D 64 102 -> 104; 2048 (1024) 332
+// -> 306, D 64 181 -> 167; 4096 (2048) 1164 -> 1155, D 64 630 -> 626.  Every odd round light
+// first: 2048 329, 4096 1173; rounds of two per CU: 1536 213, 2048 369, 4096 1148.
+__device__ __forceinline__ uint32_t prefill_f32_item(uint32_t w, uint32_t total, uint32_t cus) {
+  if (w / cus != 1) return w;
+  const uint32_t n = min(cus, total - cus), l = w - cus;
+  const uint32_t step = total % 8 == 0 && cus % 8 == 0 ? 8 : 1;
+  return cus + (n / step - 1 - l / step) * step + l % step;
 }
 
 // Library kernel: grid = batch * nh * ceil(S / 64), S >= 1; heavy query blocks first (but for
@@ -578,9 +582,9 @@ __global__ void __launch_bounds__(pf32::NT, 2)
 attn_prefill_f32(const float* __restrict__ Q, const float* __restrict__ K,
                  const float* __restrict__ V, float* __restrict__ O, uint32_t batch, uint32_t S,
                  uint32_t start_pos, uint32_t max_seq, uint32_t nh, uint32_t nkv,
-                 float scale_log2) {
+                 float scale_log2, uint32_t cus) {
   uint32_t bh, qb;
-  prefill_work(prefill_f32_item(blockIdx.x, gridDim.x), batch, nh, nkv,
+  prefill_work(prefill_f32_item(blockIdx.x, gridDim.x, cus), batch, nh, nkv,
                (S + pf32::BQ - 1) / pf32::BQ, bh, qb);
   prefill_f32_tile<D>(Q, K, V, O, S, start_pos, max_seq, nh, nkv, scale_log2, bh / nh, bh % nh,
                       qb);

@@ -533,11 +533,11 @@ int th_attention_prefill(const void* q, const void* k, const void* v, void* o, u
     if (head_dim == 64)
       hipLaunchKernelGGL(th::attn_prefill_f32<64>, grid, block, 0, as_stream(s), Q, K, V, O, batch,
                          seq_len, start_pos, max_seq, num_heads, num_kv_heads,
-                         scale * th::kLog2e);
+                         scale * th::kLog2e, current_cu_count());
     else
       hipLaunchKernelGGL(th::attn_prefill_f32<128>, grid, block, 0, as_stream(s), Q, K, V, O,
                          batch, seq_len, start_pos, max_seq, num_heads, num_kv_heads,
-                         scale * th::kLog2e);
+                         scale * th::kLog2e, current_cu_count());
     return launch_status("attention_prefill (fp32 MFMA) launch");
   }
   return attn_general_launch(q, k, v, o, batch, seq_len, start_pos, max_seq, start_pos + seq_len,
