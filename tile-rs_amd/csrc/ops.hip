@@ -80,9 +80,7 @@ bool row_wg_pays(uint32_t rows, uint32_t cols, int esz, uint32_t ps, const void*
   return rounds * cols * ps <= 2400000 + 2 * rows * bytes * 1000 / 4000;   // picoseconds
 }
 
-// The row-per-workgroup kernel's size: launch(threads, vectors per thread).  A finer last step
-// gains nothing: 13 vectors per thread against 16, softmax 256 x 50257 f32 20.3 us both, 1024 x
-// 33001 55.3 and 55.5.
+// The row-per-workgroup kernel's size: launch(threads, vectors per thread).
 template <class F>
 void row_wg_by_size(uint32_t cols, int esz, F&& launch) {
   const uint32_t vec = (cols * static_cast<uint32_t>(esz) + 15) / 16;
@@ -93,6 +91,7 @@ void row_wg_by_size(uint32_t cols, int esz, F&& launch) {
   else if (vec <= 1024 * 2) go(integral_constant<int, 1024>{}, integral_constant<int, 2>{});
   else if (vec <= 1024 * 4) go(integral_constant<int, 1024>{}, integral_constant<int, 4>{});
   else if (vec <= 1024 * 8) go(integral_constant<int, 1024>{}, integral_constant<int, 8>{});
+  else if (vec <= 1024 * 13) go(integral_constant<int, 1024>{}, integral_constant<int, 13>{});
   else go(integral_constant<int, 1024>{}, integral_constant<int, 16>{});
 }
 
