@@ -21,7 +21,8 @@
  *     of check_cu in crates/tile_hal/src/cuda.rs:124-130.
  *   - No function throws across this boundary and none takes torch types.
  *   - Streams are HIP streams (hipStream_t) passed as void*; NULL means the
- *     default stream of the current device.
+ *     default stream of the current device, hipStreamPerThread the calling
+ *     thread's (library scratch there is the thread's own).
  *   - 16-bit floats (f16 and bf16) share the uint16_t carrier, as in tile_std
  *     (crates/tile_std/src/lib.rs:182); a th_dtype tag says which.
  */
@@ -225,7 +226,8 @@ int th_attention_decode(const void* q, const void* k, const void* v, void* o, ui
 /* th_attention_decode that allocates nothing.  No counterpart in the reference:
  * it is for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc).  Same result
- * as th_attention_decode.  The split partials go to a fixed 8 MiB array in each
+ * as th_attention_decode, bit for bit in 16 bits; f32 runs on the general kernel,
+ * unsplit, so it is slower and its sums run in another order.  The split partials go to a fixed 8 MiB array in each
  * GPU's memory that is loaded with the library's code object and held until the
  * process ends; a plan whose partials would need more returns TH_MEMORY_ERROR,
  * and head dims below 128 other than 64 (which run on padded copies) return

@@ -121,3 +121,20 @@ def test_decode_f32_shapes(dev, stream, B, L, extra, NH, NKV, Dh, ws):
     assert err < 1e-5, f"max err {err:.3e}"
     if wb is not None:
         assert (wb.copy_to_host(stream)[size // 4:] == 3.0).all()
+
+
+@pytest.mark.parametrize("B,L,NH,NKV,Dh", [(1, 3000, 8, 2, 128), (2, 700, 4, 4, 64)])
+def test_decode_static_f32(dev, stream, B, L, NH, NKV, Dh):
+    """f32 without allocation: the general kernel, close to the split kernel's result."""
+    rng = np.random.default_rng(L)
+    q = rng.standard_normal((B, NH, Dh)).astype(np.float32)
+    k, v = (rng.standard_normal((B, NKV, L, Dh)).astype(np.float32) for _ in range(2))
+    bufs = [put(dev, stream, x) for x in (q, k, v)]
+    out = [put(dev, stream, np.full(q.size, 7.0, np.float32)) for _ in range(2)]
+    th.attention_decode(*bufs, out[0], B, L, L, Dh, NH, NKV, D.F32, None, 0, stream)
+    th._lib.check(th.lib().th_attention_decode_static(
+        *(b.as_raw_ptr() for b in bufs), out[1].as_raw_ptr(), B, L, L, Dh, NH, NKV, int(D.F32),
+        stream.handle))
+    got, static = (o.copy_to_host(stream).reshape(q.shape) for o in out)
+    ref = orc.attention_decode(q, k, v, orc.F32, B, L, L, Dh, NH, NKV).reshape(q.shape)
+    assert np.abs(got - ref).max() < 1e-5 and np.abs(static - ref).max() < 1e-5

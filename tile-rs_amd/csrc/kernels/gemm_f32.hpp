@@ -185,7 +185,8 @@ gemm_f32_mfma(const float* __restrict__ A, const float* __restrict__ B, void* __
 // writes, whose 16 lane groups then read 64 consecutive bytes of a matrix row each.
 //
 // Measured on MI355X: 999 x 4096 x 1000 522 -> 91 us (90 TFLOP/s), 1024^3 96 -> 27,
-// 300 x 3000 x 500 397 -> 21, 64 x 4096 x 64 427 -> 10.
+// 300 x 3000 x 500 397 -> 21, 64 x 4096 x 64 427 -> 10.  Counters at 999 x 4096 x 1000: MFMA
+// busy 56%, 1.6 LDS instructions per MFMA, 14% of the LDS-active cycles in bank conflicts.
 // ============================================================================
 namespace gf32s {
 constexpr int BM = 64, BN = 64, BK = 64;

@@ -1,7 +1,7 @@
 // GEMM entry points of the C ABI (include/tilers_hip.h, section 2): th_matmul and
-// th_matmul_silu_mul, and their kernels for 16-bit operands (f32: ops_gemm_f32.hip).  Shapes and pointers are checked on the host, the hand-written
-// gfx950 kernel for the shape is picked and enqueued on the caller's stream; there is
-// no CPU fallback.  (Its own translation unit: the GEMM instantiations compile in
+// th_matmul_silu_mul, and their kernels for 16-bit operands (f32: ops_gemm_f32.hip).
+// Shapes and pointers are checked on the host, the hand-written gfx950 kernel for the
+// shape is picked and enqueued on the caller's stream; there is no CPU fallback.  (Its own translation unit: the GEMM instantiations compile in
 // parallel with the rest of the library.)
 #include <hip/hip_runtime.h>
 

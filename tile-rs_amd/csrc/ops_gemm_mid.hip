@@ -44,7 +44,7 @@ int go(const GemmArgs& g, th_dtype out, GemmPlan p) {
   // No split without memory for the partials.  While a graph is recorded (nothing can be
   // allocated, and its replays could meet on the stream's scratch): only in place of a split
   // on 256 x 256 tiles, which shares that buffer too, and if it is large enough already.
-  // (Row-major B 8 x 14336 x 4096 needs it: 64 workgroups unsplit.)
+  // (Row-major B 8 x 4096 x 1024 needs it: 16 workgroups unsplit.)
   const uint64_t bytes = static_cast<uint64_t>(p.slices) * g.m * g.n * sizeof(float);
   if (p.slices > 1 &&
       ((stream_capturing(g.s) && !(p.in_graph && th::stream_scratch_ready(g.s, bytes))) ||
@@ -75,12 +75,14 @@ int go(const GemmArgs& g, th_dtype out, GemmPlan p) {
 //   register-staged one 155;
 //   128 x 64 tiles max(30.5, 4 + 22.5 w), 64 x 64 tiles max(20.5, 5 + 13.5 w), w tiles per CU
 //   (row-major B 1.12 times, rows off 128 bytes 1.3, B over 64 MB 1.08 to 1.4), no faster than
-//   A and B come in at 3 TB/s;
+//   A and B come in at 3 TB/s (a line for these tiles alone: split 256 x 256 ones stream B
+//   at 5.2 TB/s, row-major 8 x 14336 x 4096 22.4 against 23.9 at the best split of 64 x 64);
 //   a K split adds 4 us and its f32 partials, written and read at 4 TB/s.
-// E.g. (bf16, row-major, us, against 256 x 256 tiles with K split until the chip is full) 100
-// x 4096 x 4096 23 -> 19, 1000 x 4096 x 1024 38 -> 24, 4096 x 4096 x 1024 73 -> 46, 512 x 4096
-// x 4096 44 -> 37, 1000 x 4096 x 4096 72 -> 50, 2048 x 4096 x 4096 103 -> 71 (256 x 256, no
-// split), 300 x 3752 x 2840 144 -> 23.
+// E.g. (bf16, row-major, us, one box, against 256 x 256 tiles always, K split in as many equal
+// slices of whole stages as give no CU two workgroups) 100 x 4096 x 4096 30 -> 18, 1000 x 4096 x
+// 1024 53 -> 24, 4096 x 4096 x 1024 71 -> 47, 512 x 4096 x 4096 59 -> 36, 1000 x 4096 x 4096
+// 71 -> 47, 2048 x 4096 x 4096 102 -> 65 (256 x 256, no split), 300 x 3752 x 2840 143 -> 22, 8 x
+// 4096 x 1024 12.7 -> 7.9.
 GemmPlan plan_16bit(const GemmArgs& g, const GemmForms& f) {
   const double cus = current_cu_count(), mn = static_cast<double>(g.m) * g.n;
   const double kk = g.k / 4096.0;
